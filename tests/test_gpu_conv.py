@@ -56,6 +56,31 @@ def test_conv_batch_equals_steps_and_state(gpu):
     C.free()
 
 
+@pytest.mark.parametrize("dim,T", [(64, 2), (1000, 3), (1004, 5), (2056, 4), (1024, 513)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_conv_batch_shapes(gpu, dim, T, shift):
+    """A batch's parallel kernel at one- and eight-channel widths, odd and even
+    batches, rows that do and do not start on 16 bytes; then the in-place form
+    (y over bcx), which walks the positions."""
+    import torch
+    rng = np.random.default_rng(dim + T)
+    w, bcx = _case(rng, 1, dim, T + 1)
+    taps = o.conv_taps(w[0])
+    st = np.zeros((2, dim), np.int16)
+    want = np.stack([o.conv_step(bcx[t], taps, st) for t in range(T + 1)])
+    for inplace in (False, True):
+        C = gpu.conv(w)
+        first = host(C.step(0, dev(bcx[0])))
+        buf = torch.zeros(T * 3 * dim + shift, dtype=torch.int16, device="cuda")
+        x = buf[shift:].view(T, 3 * dim)
+        x.copy_(dev(bcx[1:]))
+        out = buf[shift:shift + T * dim].view(T, dim) if inplace else None
+        got = host(C.step(0, x, out=out))
+        assert np.array_equal(np.concatenate([first[None], got]), want)
+        assert np.array_equal(C.state(0), st)
+        C.free()
+
+
 def test_conv_refusals(gpu):
     from vgx.lib import VgxError
     w = np.zeros((2, 64, 3), np.float32)

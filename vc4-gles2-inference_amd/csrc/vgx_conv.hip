@@ -11,7 +11,9 @@
 // (engine/src/shaders.cpp:1991-2051), fp32 in the shaders' order, operands of
 // conv3 in q16 units, taps = q16 of the f32 kernel (set_conv_kernel,
 // engine/src/gpu_conv.cpp:84-101).  The state is the last two gated values
-// per layer.  One thread per channel walks the batch in position order, so a
+// per layer.  A position needs only its own gated value and the two before it,
+// and a gated value needs only its own row of bcx, so a batch's positions run
+// in parallel, each thread recomputing the two gated values before its run: a
 // batch of n positions equals n single steps.
 //
 // HBM layout: taps [layers][3][dim] int16, state [layers][2][dim] int16
@@ -67,6 +69,78 @@ __global__ void __launch_bounds__(kThreads) conv_kernel(int dim, int ntok, const
     }
     state[i] = (int16_t)s2;
     state[dim + i] = (int16_t)s1;
+}
+
+// A batch, in parallel over positions: a thread takes V channels (V = 8: one
+// 16-byte load a row) of kRun consecutive positions.  Every load of the run is
+// issued at once from clamped rows (one memory round trip), where conv_kernel
+// has a dependent round trip a position: 200 positions of 1,024 channels
+// 72.5 -> 3.8 us (bound by that one round trip and the launch; the two rows
+// each run reads again come from the L2).  kRun = 2: with more positions a
+// thread the loads of a run are fewer per output, but a batch has too few waves.
+// The state is read and written by the first run's threads alone (they form
+// the last two gated values themselves), so no workgroup reads what another
+// writes.
+constexpr int kRun = 2;
+
+template <int V>
+struct __align__(2 * V) Vec {
+    int16_t v[V];
+};
+
+template <int V>
+__global__ void __launch_bounds__(kThreads) conv_batch_kernel(int dim, int ntok, const int16_t* bcx,
+                                                              const int16_t* taps, int16_t* state, int16_t* y) {
+    using T = Vec<V>;
+    const int i = (blockIdx.x * blockDim.x + threadIdx.x) * V;
+    if (i >= dim) return;
+    const int t0 = blockIdx.y * kRun;
+    auto at = [&](const int16_t* p) { return *reinterpret_cast<const T*>(p); };
+    auto row = [&](int t) { return bcx + (size_t)min(max(t, 0), ntok - 1) * 3 * dim + i; };
+    T b[kRun + 2], x[kRun + 2], c[kRun], lb[2], lx[2], old[2];
+#pragma unroll
+    for (int k = 0; k < kRun + 2; ++k) {
+        b[k] = at(row(t0 - 2 + k));
+        x[k] = at(row(t0 - 2 + k) + 2 * dim);
+    }
+#pragma unroll
+    for (int k = 0; k < kRun; ++k) c[k] = at(row(t0 + k) + dim);
+    const T k0 = at(taps + i), k1 = at(taps + dim + i), k2 = at(taps + 2 * dim + i);
+    if (t0 == 0) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            old[k] = at(state + (size_t)k * dim + i);
+            lb[k] = at(row(ntok - 2 + k));
+            lx[k] = at(row(ntok - 2 + k) + 2 * dim);
+        }
+    }
+    T o[kRun];
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+        auto gated = [](int16_t bv, int16_t xv) { return q16_store((float)bv / 256.0f * ((float)xv / 256.0f)); };
+        int s2 = t0 == 0 ? (int)old[0].v[e] : gated(b[0].v[e], x[0].v[e]);
+        int s1 = t0 == 0 ? (int)old[1].v[e] : gated(b[1].v[e], x[1].v[e]);
+#pragma unroll
+        for (int k = 0; k < kRun; ++k) {
+            const int g = gated(b[k + 2].v[e], x[k + 2].v[e]);
+            const float acc = (((float)k0.v[e] * (float)s2 + (float)k1.v[e] * (float)s1) + (float)k2.v[e] * (float)g) *
+                              0.00390625f;
+            o[k].v[e] = (int16_t)q16_store((float)c[k].v[e] / 256.0f * ((float)q16_round(acc) / 256.0f));
+            s2 = s1;
+            s1 = g;
+        }
+        if (t0 == 0) {  // (ntok >= 2)
+            lb[0].v[e] = (int16_t)gated(lb[0].v[e], lx[0].v[e]);
+            lb[1].v[e] = (int16_t)gated(lb[1].v[e], lx[1].v[e]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kRun; ++k)
+        if (t0 + k < ntok) *reinterpret_cast<T*>(y + (size_t)(t0 + k) * dim + i) = o[k];
+    if (t0 == 0) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) *reinterpret_cast<T*>(state + (size_t)k * dim + i) = lb[k];
+    }
 }
 
 // zero fill by a kernel (safe inside a captured graph)
@@ -143,6 +217,25 @@ int vgx_conv_step(vgx_conv* c, int layer, int ntok, const int16_t* bcx, int16_t*
     VGX_HIP(hipSetDevice(c->ctx->device));
     const int16_t* taps = c->taps + (size_t)layer * 3 * c->dim;
     int16_t* st = c->state + (size_t)layer * 2 * c->dim;
+    // A batch runs its positions in parallel, 8 channels a thread where every
+    // row starts on 16 bytes.  One position, and rows written over bcx (each
+    // channel's walk reads a value before it is overwritten), keep the walk.
+    const size_t yn = (size_t)ntok * c->dim;
+    const bool apart = y + yn <= bcx || bcx + 3 * yn <= y;
+    const unsigned runs = ((unsigned)ntok + kRun - 1) / kRun;
+    if (ntok > 1 && apart && runs <= 65535u) {
+        const bool wide = c->dim % 8 == 0 && (((uintptr_t)bcx | (uintptr_t)y) & 15u) == 0;
+        const int per = wide ? c->dim / 8 : c->dim;
+        // whole waves, no more than the channels need
+        const int nt = per < kThreads ? (per + 63) / 64 * 64 : kThreads;
+        const dim3 grid((per + nt - 1) / nt, runs);
+        if (wide)
+            hipLaunchKernelGGL(conv_batch_kernel<8>, grid, dim3(nt), 0, c->ctx->stream, c->dim, ntok, bcx, taps, st, y);
+        else
+            hipLaunchKernelGGL(conv_batch_kernel<1>, grid, dim3(nt), 0, c->ctx->stream, c->dim, ntok, bcx, taps, st, y);
+        VGX_LAUNCH_CHECK("conv batch launch");
+        return VGX_OK;
+    }
     hipLaunchKernelGGL(conv_kernel, dim3((c->dim + kThreads - 1) / kThreads), dim3(kThreads), 0, c->ctx->stream,
                        c->dim, ntok, bcx, taps, st, y);
     VGX_LAUNCH_CHECK("conv launch");
