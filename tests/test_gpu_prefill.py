@@ -102,6 +102,90 @@ def test_ffn_gate_batch(gpu, kind, rows, cols):
             assert np.array_equal(got[t], want), (hs, t)
 
 
+# The tile kernel's plans by output tiles of 32 x 32 (rows/32 x tokens/32: up to
+# one a CU, 2.2, 3.5, 6 and more at 256 CUs), with ragged rows and tokens, a row of
+# one k-step and rows that end inside a k tile, past one K group's run or before
+# the last group's; the split column off a k-step where the format allows it.
+@pytest.mark.parametrize("kind", ["q8", "q4", "t3"])
+@pytest.mark.parametrize("rows,ntok", [(33, 33), (2100, 70), (4130, 97), (6150, 97), (9650, 97), (13000, 129)])
+@pytest.mark.parametrize("cols_unit", [1, 3, 19])
+def test_gemm_tile_plans(gpu, kind, rows, ntok, cols_unit):
+    rng = np.random.default_rng(rows + ntok + cols_unit)
+    cols = cols_unit * {"q8": 16, "q4": 32, "t3": 8}[kind]
+    m1, m3 = MK[kind](rng, rows, cols), MK[kind](rng, rows, cols)
+    W1, W3 = gpu.upload(m1), gpu.upload(m3)
+    x = x_rows(rng, ntok, cols)
+    x[0], x[-1] = 32767, -32768
+    res = x_rows(rng, ntok, rows)
+    X, R = dev(x), dev(res)
+    got, got_r, gate = host(gpu.gemm(W1, X)), host(gpu.gemm(W1, X, res=R)), host(gpu.ffn_gate_batch(W1, W3, X, 1))
+    unit = {"q8": 16, "q4": 32, "t3": 32}[kind]
+    split = cols // 2 // unit * unit
+    got_s = host(gpu.gemm_add_split(W1, split, X, R)) if split else None
+    for t in {0, 1, 31, 32, ntok // 2, ntok - 1}:
+        v = oracle_rowval(m1, x[t])
+        assert np.array_equal(got[t], o.store(v)), t
+        assert np.array_equal(got_r[t], o.store(v, res[t])), t
+        assert np.array_equal(gate[t], o.gate(v, oracle_rowval(m3, x[t]), 1)), t
+        if split:
+            y1 = o.store(oracle_rowval(m1.slice_cols(0, split), x[t, :split]), res[t])
+            assert np.array_equal(got_s[t], o.store(oracle_rowval(m1.slice_cols(split, cols), x[t, split:]), y1)), t
+    # the tokens between: the batch equals itself in other batch sizes
+    for t0 in range(0, ntok, 32):
+        assert np.array_equal(got[t0:t0 + 32], host(gpu.gemm(W1, dev(x[t0:t0 + 32]))))
+        assert np.array_equal(gate[t0:t0 + 32], host(gpu.ffn_gate_batch(W1, W3, dev(x[t0:t0 + 32]), 1)))
+
+
+@pytest.mark.parametrize("kind", ["q8", "q4", "t3"])
+def test_gemm_sums_past_24_bits(gpu, kind):
+    """Sums whose halves are not exact floats (the epilogue's 64-bit form): rows
+    at the rails beside ordinary ones."""
+    rng = np.random.default_rng(11)
+    rows, cols, ntok = 96, 4096, 70
+    m = MK[kind](rng, rows, cols)
+    if kind == "q8":
+        m.body.reshape(rows, cols)[::2] = 255
+    elif kind == "q4":
+        m.body.reshape(rows, cols // 2)[::2] = 0xFF
+        m.s16.reshape(rows, -1)[::2] = 32767
+        m.m16.reshape(rows, -1)[::2] = 32767
+    m.scale *= 1e-4
+    W = gpu.upload(m)
+    x = x_rows(rng, ntok, cols)
+    x[::3] = 32767
+    x[1::3] = -32768
+    for split in (0, cols // 2):
+        res = x_rows(rng, ntok, rows)
+        got = host(gpu.gemm_add_split(W, split, dev(x), dev(res)) if split else gpu.gemm(W, dev(x), res=dev(res)))
+        for t in range(ntok):
+            want = res[t]
+            for a, b in ([(0, split), (split, cols)] if split else [(0, cols)]):
+                want = o.store(oracle_rowval(m.slice_cols(a, b), x[t, a:b]), want)
+            assert np.array_equal(got[t], want), (split, t)
+
+
+@pytest.mark.parametrize("chunk", [32, 8192, 65536])
+def test_gate_every_input(gpu, chunk):
+    """The batched gate's table exponential and refined quotient at every one
+    of the 65,536 gate values, against the oracle's exp and division, for
+    several up values and hidden exponents."""
+    from vgx import mmcf
+    rows, cols = 32, 16
+    lev = np.zeros((2, rows, cols), np.uint8) + 128
+    lev[0, :, 0] += 1   # W1: x[0]
+    lev[1, :, 1] += 1   # W3: x[1]
+    W1, W3 = (gpu.upload(mmcf.Matrix("q8", rows, cols, l.ravel(), 1.0, True, None)) for l in lev)
+    g = np.arange(-32768, 32768).astype(np.int16)
+    if chunk == 32:  # one token tile: a sample of them
+        g = g[::997]
+    for up, hs in ((32767, 0), (-32768, 0), (300, 0), (7777, 5)):
+        x = np.zeros((g.size, cols), np.int16)
+        x[:, 0], x[:, 1] = g, up
+        got = np.concatenate([host(gpu.ffn_gate_batch(W1, W3, dev(x[a:a + chunk]), hs)) for a in range(0, g.size, chunk)])
+        want = o.gate(g.astype(np.float32), np.full(g.size, up, np.float32), hs)
+        assert np.array_equal(got, np.repeat(want[:, None], rows, 1)), (up, hs)
+
+
 @pytest.mark.parametrize("kind,rows,cols,ntok", [("t3", 1280, 1024, 32), ("q8", 1536, 768, 256), ("q4", 1536, 768, 37),
                                                  ("q8", 3072, 1024, 5), ("t3", 33, 96, 32), ("q8", 73, 64, 40)])
 def test_gemm_rms(gpu, kind, rows, cols, ntok):

@@ -83,10 +83,11 @@ int vgx_ctx_create(int device, vgx_ctx** out) {
     c->device = device;
     c->num_cu = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
     c->scratch_keys = keys;
-    hipError_t e = hipStreamCreate(&c->own);
+    hipError_t e = vgx_gemm_tile_init(c->num_cu);
+    if (e == hipSuccess) e = hipStreamCreate(&c->own);
     if (e != hipSuccess) {
         delete c;
-        return vgx_hip_fail(e, "hipStreamCreate");
+        return vgx_hip_fail(e, "vgx_ctx_create");
     }
     c->stream = c->own;
     *out = c;

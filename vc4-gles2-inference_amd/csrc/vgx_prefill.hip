@@ -1,5 +1,7 @@
-// Batched prefill on the int8 matrix cores: Y[t] = W . X[t] for ntok token
-// rows at once, the same exact integer sums as the batch-1 GEMV, so every
+// Batched GEMM entry points, and the one-token-tile kernel behind the launches
+// that vgx_gemm.hip's tile kernel does not take: the RMSNorm-fused variants,
+// and q4 over at most 32 tokens (the decode of a batch).  Y[t] = W . X[t] for
+// ntok token rows with the exact integer sums of the batch-1 GEMV, so every
 // output row is bit-identical to vgx_gemv on that token (the reference's
 // acceptance rule for a batched path: the logits of a grouped prefill equal
 // the serial ones byte for byte, docs/prefill-batching.md:98-113;
@@ -36,52 +38,14 @@
 // variants normalise the activation rows on the way into LDS, with the
 // statistics formed in the workgroup (GPU::rmsnorm's rounding).
 #include <algorithm>
-#include <cmath>
 #include <mutex>
 #include <string>
 
-#include "vgx_internal.h"
-#include "vgx_qrow.h"
+#include "vgx_gemm.h"
 
 #pragma clang fp contract(off)
 
 namespace {
-
-typedef signed char i8x16 __attribute__((ext_vector_type(16)));
-typedef int i32x16 __attribute__((ext_vector_type(16)));
-
-constexpr int kTile = 32;  // tokens and weight rows per wave tile
-
-enum BatchEpi { BEPI_STORE = 0, BEPI_GATE = 1, BEPI_SPLIT = 2 };
-
-struct GemmLaunch {
-    MatDev M, M3;           // W (and W3 for the gate)
-    int ntok, cols;
-    const int16_t* x;       // ntok rows of cols q16 values, row stride ldx
-    int ldx;
-    const int16_t* res;     // residual rows (stride ldy) or nullptr
-    int16_t* y;             // ntok rows of M.rows q16 values, row stride ldy
-    int ldy;
-    int hs;                 // gate: hidden store exponent
-    int split;              // split: first column of the second half
-    const int16_t* rw;      // RMS prologue: the q16 norm weight (cols values)
-    float eps;              // RMS prologue: epsilon
-    long long* part;        // split K: [split][set][ntok][rows] exact partial sums
-    int nz;                 // split K: the launch's splits (its grid's z; from here, not from
-                            // gridDim.z, an implicit argument whose load would delay the first weights)
-};
-
-union Op {
-    i8x16 v;
-    uint32_t d[4];
-};
-
-
-
-__device__ __forceinline__ i32x16 mfma(const Op& a, const Op& b, const i32x16& c) {
-    return __builtin_amdgcn_mfma_i32_32x32x32_i8(a.v, b.v, c, 0, 0, 0);
-}
-
 
 // A operands: 16 q16 activations (two 16-byte loads of one token row) as the
 // high-byte plane and the low-byte plane minus 128; xsum = their exact sum.
@@ -100,17 +64,6 @@ __device__ __forceinline__ void x_planes(const uint4 a, const uint4 b, bool ok, 
         sl = __builtin_amdgcn_udot4(lo, 0x01010101u, sl, false);
     }
     xsum = ok ? 256 * sh + (int)sl : 0;
-}
-
-// Four 2-bit t3 codes (one byte, code j at bits 2j..2j+1) as four int8
-// levels: bit 0 = |level|, bit 1 = sign (engine/tools/mmcf_hf.py:168-199);
-// code 2 (a sign without magnitude) is level 0.  Each code is spread to its
-// own byte, then level = |l| ^ ((sign & |l|) * 0xFE): 0x01 or 0xFF.
-__device__ __forceinline__ uint32_t t3_levels(uint32_t b) {
-    const uint32_t x = (b | (b << 6) | (b << 12) | (b << 18)) & 0x03030303u;
-    const uint32_t m = x & 0x01010101u;
-    const uint32_t sg = (x >> 1) & m;
-    return m ^ (sg * 0xFEu);
 }
 
 // The bytes of weight row n, columns k0..k0+15: 16 (q8) or 8 (q4, t3, in .x
@@ -159,17 +112,6 @@ __device__ __forceinline__ void w_planes(const uint4 v, int n, bool ok, Op& w, i
 #pragma unroll
     for (int i = 0; i < 4; ++i) s = sdot4(w.d[i], 0x01010101u, s);
     wsum = s;
-}
-
-__device__ __forceinline__ float gate_value(float v1, float v3, int hs) {
-    const float g = (float)q16_round(v1), uu = (float)q16_round(v3);
-    const float a = g / 256.0f;
-    const float e = (float)exp(-(double)a);
-    const float dn = 1.0f + e;
-    const float r = a / dn;
-    float o = r * (uu / 256.0f);
-    o = o * ldexpf(1.0f, -hs);
-    return o * 256.0f;
 }
 
 // The inverse RMS of each of the workgroup's token rows (rms_stats_split,
@@ -647,25 +589,32 @@ __global__ void __launch_bounds__(kNormThreads) gemm_epi_norm_kernel(const GemmL
 
 using GemmFn = void (*)(const GemmLaunch);
 
+// The RMS variants in every format; without RMS, q4 of one token tile (whole
+// or split) and the shapes past the tile kernel's limits (4 waves).
 template <int EPI, int NW, bool RMS, bool PART>
 GemmFn pick_kind(int kind) {
     switch (kind) {
-        case VGX_Q8: return gemm_kernel<VGX_Q8, EPI, NW, RMS, PART>;
+        case VGX_Q8: return PART ? nullptr : gemm_kernel<VGX_Q8, EPI, NW, RMS, false>;
         case VGX_Q4: return gemm_kernel<VGX_Q4, EPI, NW, RMS, PART>;
-        case VGX_T3: return gemm_kernel<VGX_T3, EPI, NW, RMS, PART>;
+        case VGX_T3: return PART ? nullptr : gemm_kernel<VGX_T3, EPI, NW, RMS, false>;
     }
     return nullptr;
 }
 
 template <int EPI, bool RMS>
 GemmFn pick_nw(int kind, int nw, bool part) {
-    if (part) return nw == 4 ? pick_kind<EPI, 4, RMS, true>(kind) : nullptr;
-    switch (nw) {
-        case 2: return pick_kind<EPI, 2, RMS, false>(kind);
-        case 4: return pick_kind<EPI, 4, RMS, false>(kind);
-        case 8: return pick_kind<EPI, 8, RMS, false>(kind);
+    if constexpr (RMS) {
+        switch (nw) {
+            case 2: return pick_kind<EPI, 2, true, false>(kind);
+            case 4: return pick_kind<EPI, 4, true, false>(kind);
+            case 8: return pick_kind<EPI, 8, true, false>(kind);
+        }
+        return nullptr;
+    } else {
+        if (part) return kind == VGX_Q4 ? pick_kind<EPI, 4, false, true>(kind) : nullptr;
+        if (nw == 8) return kind == VGX_Q4 ? gemm_kernel<VGX_Q4, EPI, 8, false, false> : nullptr;
+        return nw == 4 ? pick_kind<EPI, 4, false, false>(kind) : nullptr;
     }
-    return nullptr;
 }
 
 GemmFn pick(int epi, int kind, int nw, bool rms, bool part) {
@@ -765,10 +714,15 @@ int launch(vgx_ctx* ctx, const vgx_mat* W, const vgx_mat* W3, int ntok, const in
     L.split = split;
     L.rw = rw;
     L.eps = eps;
+    if (!rw) {
+        // (VGX_ESTATE: a launch the tile kernel leaves to this file's)
+        const int st = vgx_gemm_tile_launch(L, epi, ctx->num_cu, ctx->stream);
+        if (st != VGX_ESTATE) return st || !yn ? st : vgx_rmsnorm_batch(ctx, ntok, M.rows, y, nrm_w, neps, yn);
+    }
     dim3 grid((M.rows + kTile - 1) / kTile, (ntok + kTile - 1) / kTile);
     const int nsteps = (M.cols + kTile - 1) / kTile;
     // (the RMS variants stay whole: every split would recompute the row statistics)
-    int nz = rw ? 1 : k_splits((int)grid.x, (int)grid.y, nsteps, ctx->num_cu);
+    int nz = rw || M.kind != VGX_Q4 ? 1 : k_splits((int)grid.x, (int)grid.y, nsteps, ctx->num_cu);
     if (nz > 1) {
         const int na = epi == BEPI_STORE ? 1 : 2;
         const size_t bytes = (size_t)nz * na * ntok * M.rows * sizeof(long long);
@@ -776,7 +730,8 @@ int launch(vgx_ctx* ctx, const vgx_mat* W, const vgx_mat* W3, int ntok, const in
         grid.z = nz;
     }
     L.nz = nz;
-    const int nw = nz > 1 ? 4 : waves_for((int)(grid.x * grid.y), nsteps, ctx->num_cu);
+    int nw = nz > 1 ? 4 : waves_for((int)(grid.x * grid.y), nsteps, ctx->num_cu);
+    if (!rw && (M.kind != VGX_Q4 || nw == 2)) nw = 4;  // (the variants that exist without RMS)
     GemmFn fn = pick(epi, M.kind, nw, rw != nullptr, nz > 1);
     if (!fn) return vgx_fail(VGX_EINVAL, std::string(who) + ": unknown weight kind");
     // each wave's activation block (32 tokens x 4 k-steps of 32 int16), then
