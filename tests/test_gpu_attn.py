@@ -283,3 +283,79 @@ def test_query_block_sequences(gpu, bits, heads, kvh, hd, seq):
     for s in range(nseq):
         assert np.array_equal(A.view(s).read_rows(0, 0, seq), kv[s]), s
     A.free()
+
+
+# The tile kernel (8 or more query vectors a workgroup): query vectors of 8, 16,
+# 32, 3, 1 and 2 heads a KV head, head_dim of one to eight element tiles (one and
+# two 64-wide key steps, the second padded), batches that end inside a block,
+# contexts around a chunk and a round of four chunks, cached rows at the rails.
+# (bits, heads, kv_heads, head_dim, seq, (pos0, rows) ..., rails)
+TILE = [(16, 8, 1, 64, 320, ((0, 2), (30, 3), (100, 29), (191, 129)), False),
+        (8, 8, 1, 64, 320, ((0, 2), (30, 3), (100, 29), (191, 129)), False),
+        (16, 16, 1, 16, 160, ((0, 33), (60, 5), (126, 34)), False),
+        (8, 32, 1, 32, 160, ((0, 33), (95, 2), (126, 34)), True),
+        (16, 48, 16, 48, 96, ((0, 40), (31, 41)), False),
+        (8, 64, 64, 16, 96, ((0, 33), (60, 36)), False),
+        (16, 64, 32, 96, 300, ((0, 37), (257, 43)), False),
+        (8, 64, 32, 96, 300, ((0, 37), (257, 43)), False),
+        (16, 16, 2, 128, 160, ((0, 17), (120, 40)), True),
+        (8, 16, 2, 128, 160, ((0, 17), (120, 40)), True),
+        (16, 16, 2, 64, 160, ((0, 17), (120, 40)), True)]
+
+
+@pytest.mark.parametrize("bits,heads,kvh,hd,seq,batches,rails", TILE)
+def test_tile_attention_batches(gpu, bits, heads, kvh, hd, seq, batches, rails):
+    dim, width = heads * hd, heads * hd + 2 * kvh * hd
+    rng = np.random.default_rng(bits + heads * hd + kvh)
+    rc, rs = o.rope_cos_sin(10000.0, hd, seq)
+    rtab = o.rope_table(rc, rs)
+    qk = 0 if rails else 1
+    qn = rng.uniform(0.5, 1.5, (1, hd)).astype(np.float32) if qk else None
+    kn = rng.uniform(0.5, 1.5, (1, hd)).astype(np.float32) if qk else None
+    A = gpu.attention(dim=dim, heads=heads, kv_heads=kvh, head_dim=hd, seq=seq, layers=1, kv_bits=bits,
+                      rope_half=1, qk_norm=qk, rope_cos=rc, rope_sin=rs, q_norm=qn, k_norm=kn)
+    c = o.attn_cfg(dim, heads, kvh, hd, seq, bits, 1, qk)
+    qnq, knq = (o.quantize_act(qn[0]), o.quantize_act(kn[0])) if qk else (None, None)
+    rb = o.kv_row_bytes(c)
+    if bits == 16:
+        lo, hi = (-32768, 32767) if rails else (-6000, 6000)
+        vals = rng.choice([lo, hi], size=(seq, rb // 2)) if rails else rng.integers(lo, hi, size=(seq, rb // 2))
+        rows = vals.astype(">i2").view(np.uint8).reshape(-1)
+    else:
+        vals = rng.choice([-128, 127], size=(seq, rb)) if rails else rng.integers(-128, 128, size=(seq, rb))
+        rows = vals.astype(np.int8).view(np.uint8).reshape(-1)
+    for pos0, n in batches:
+        A.write_rows(0, 0, rows)
+        x = np.clip(rng.standard_normal((n, width)) * 600, -32768, 32767).astype(np.int16)
+        if rails:
+            x[::2] = rng.choice([-32768, 32767], size=x[::2].shape)
+        X = dev(x)
+        got = A.block_batch(0, pos0, X)
+        # every row: the per-head kernel on the same cache
+        for t in range(n):
+            assert torch.equal(A.decode(0, pos0 + t, X[t]), got[t]), (pos0, t)
+        # the first, a middle and the last row: the oracle
+        got = got.cpu().numpy()
+        for t in (0, n // 2, n - 1):
+            kv = A.read_rows(0, 0, seq).copy()  # (rows past the position are not read)
+            want = o.attn_block(c, x[t], qnq, knq, rtab, pos0 + t, kv)
+            assert np.array_equal(got[t], want), (pos0, t)
+    A.free()
+
+
+def test_exp_tables_round_as_exp():
+    """The tile kernel's exp(-k/1024) = T[k >> 8] * U[k & 255] and the batched
+    gate's exp(-g/256) = T'[(g >> 8) + 128] * U'[g & 255], as floats: over every
+    argument the exact value keeps 2^-44 away from a float rounding boundary,
+    four hundred times what two factors and a product in double can err."""
+    for x in (-np.arange(65536, dtype=np.longdouble) / 1024, -np.arange(-32768, 32768, dtype=np.longdouble) / 256):
+        e = np.exp(x)
+        with np.errstate(over="ignore"):
+            f = e.astype(np.float32)
+        up, dn = np.nextafter(f, np.float32(np.inf)), np.nextafter(f, np.float32(-np.inf))
+        ok = np.isfinite(f) & np.isfinite(up) & (f > 0) & (x != 0)
+        for nb in (up, dn):
+            mid = (f.astype(np.longdouble) + nb.astype(np.longdouble)) / 2
+            assert (np.abs(e - mid)[ok] / e[ok]).min() > 2.0 ** -44
+        # past the float range on either side by more than that
+        assert not np.any(f[~ok & (x < 0)]) and np.all(np.isinf(f[~ok & (x > 0)]) | (x[~ok & (x > 0)] > 88))

@@ -1389,6 +1389,380 @@ __global__ void __launch_bounds__(kThreads) attn_group_kernel(const AttnDev A, c
     }
 }
 
+// ---------------------------------------------------------------------------
+// Batches of positions on the matrix cores.  A workgroup holds up to 16 query
+// vectors (the heads of a KV head's group at consecutive positions) and follows
+// the per-head kernel's arithmetic value for value:
+//   scores   q . k by v_mfma_i32_16x16x64_i8 over byte planes, a wave per 16
+//            positions: the exact integer of the dot products
+//   exp      exp(-k/1024) of an integer k in 0..65535 as the product of two
+//            256-entry tables of doubles: no exp(-k/1024) lies within 2^-39 of a
+//            float rounding boundary (over all 65536), and the product is
+//            within 2^-50, so the float is the one of exp in double
+//   V        v_mfma_f64_16x16x4_f64, a wave per 16 elements: it accumulates its
+//            four positions by fused multiply-adds in position order (checked bit
+//            for bit on this part), so a chunk's eight steps are its chain from
+//            0.0, and the chunk sums add in chunk order
+// What bounds it: a workgroup's chain of phases, and in a long context the f64
+// products (64 clocks a 16 x 16 x 4 step, the vector rate; but V is converted once
+// and no weight is broadcast).  The query-block kernel before it dotted each
+// (query, position) pair on the vector units with the query read from LDS, formed
+// each exponential in double and broadcast each weight to a wave.  Measured, us a
+// launch (positions, query / KV heads of head_dim, cache): 512, 16 / 8 of 64, q16
+// 67.5 -> 20.8; 256 after 512, the same 58.2 -> 23; 256, 8 / 4 of 96, q8 19.2 ->
+// 13.6; 117, 16 / 2 of 64, q16 14.7 -> 9.0.  Of the 20.8, query preparation and
+// launch are 5.5, scores 3.7, exponentials 2.8, sums 1.2, products 7.6 with eight waves
+// (two sets of chunk pairs; four waves and one set: 22.1 in all).
+struct TileArgs {
+    const uint8_t* kv;
+    const int32_t* rtab;
+    const int16_t* qn;
+    const int16_t* qkv;
+    int16_t* out;
+    int pos0, ntok, nby;  // first position, rows, row blocks
+    int tq, hs;           // rows and query heads a workgroup (tq * hs <= 16)
+    int nw;               // waves
+    int fstride;          // floats of a query vector's score row: 33 a chunk, 4 mod 64 in all
+    int o_q, o_cq, o_max, o_cs, o_x, o_f;  // LDS byte offsets (the exp tables are at 0)
+};
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+// Global loads stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int KVB, int KS>
+__global__ void __launch_bounds__(512 * KS, 4) attn_tile_kernel(const AttnDev A, const TileArgs g) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    constexpr int HP = 64 * KS;  // a query plane row: head_dim padded with zeros
+    constexpr int NL = KVB / 8;  // 16-byte loads of 16 K values
+    const int hd = A.hd, G = A.group, kv_dim = A.kv_heads * hd, nw = g.nw, hs = g.hs;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lg = lane >> 4;
+    const int nsl = G / hs;
+    const int kvh = blockIdx.x / nsl, h0 = kvh * G + (blockIdx.x - kvh * nsl) * hs;
+    // row blocks: the longest contexts first, then the shortest up, so the
+    // workgroups that share a CU add up to about the same length
+    const int by = blockIdx.y, half = (g.nby + 1) >> 1;
+    const int rbase = (by < half ? g.nby - 1 - by : by - half) * g.tq;
+    const int nrow = min(g.tq, g.ntok - rbase), nq = hs * nrow;
+    const int pfirst = g.pos0 + rbase, npmax = pfirst + nrow;
+    const int nch = (npmax + kChunk - 1) / kChunk;
+    const uint8_t* khead = g.kv + (size_t)kvh * A.seq * A.pstride;
+    const uint8_t* vhead = g.kv + (size_t)(A.kv_heads + kvh) * A.seq * A.pstride;
+    double* const tab = reinterpret_cast<double*>(smem);  // exp(-i/4), then exp(-j/1024)
+    int8_t* const qp = reinterpret_cast<int8_t*>(smem + g.o_q);  // [2][16][HP]: q >> 8, (q & 255) - 128
+    int* const cq = reinterpret_cast<int*>(smem + g.o_cq);       // [16]
+    float* const wmax = reinterpret_cast<float*>(smem + g.o_max);  // [nw][16]
+    double* const cs = reinterpret_cast<double*>(smem + g.o_cs);   // [16][nch]
+    float* const F = reinterpret_cast<float*>(smem + g.o_f);       // [16][fstride]
+    auto npos_of = [&](int v) { return v < nq ? pfirst + v / hs + 1 : 0; };
+
+    // K rows of this wave's first chunk, 16 positions at a time (past the context:
+    // zeros; past the head: the next row's bytes, against zero query bytes)
+    const __amdgpu_buffer_rsrc_t krs = rows_rsrc(khead, npmax * A.pstride);
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 kr[2][KS][NL];
+    auto k_load = [&](int c, int b) {
+        const int off = (c * kChunk + 16 * b + li) * A.pstride + lg * 16 * NL;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int i = 0; i < NL; ++i)
+                kr[b][s][i] = __builtin_bit_cast(
+                    u32x4, __builtin_amdgcn_raw_buffer_load_b128(krs, off + s * 64 * NL + 16 * i, 0, 0));
+    };
+
+    // the query vectors' inputs: vector v = j*hs + i is row j of the block,
+    // head h0 + i; a wave takes v = wave, wave + nw, ...
+    int qa[2][KS], qb[2][KS], na[2][KS], nb[2][KS], co[2][KS], sn[2][KS];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int v = min(wave + u * nw, nq - 1), j = v / hs;
+        const int16_t* x = g.qkv + (size_t)(rbase + j) * (A.dim + 2 * kv_dim) + (h0 + v - j * hs) * hd;
+        const int32_t* rt = g.rtab + (size_t)(pfirst + j) * (hd / 2) * 2;
+#pragma unroll
+        for (int c = 0; c < KS; ++c) {
+            const int i = min(lane + 64 * c, hd - 1);
+            int jj, ti;
+            bool first;
+            rope_pair(A.rope_half, hd, i, jj, ti, first);
+            qa[u][c] = x[i];
+            qb[u][c] = x[jj];
+            na[u][c] = A.qk_norm ? g.qn[i] : 0;
+            nb[u][c] = A.qk_norm ? g.qn[jj] : 0;
+            co[u][c] = rt[2 * ti];
+            sn[u][c] = rt[2 * ti + 1];
+        }
+    }
+    k_load(wave, 0);
+    k_load(wave, 1);
+    for (int i = tid; i < 512; i += 64 * nw) tab[i] = exp(i < 256 ? -(double)i * 0.25 : -(double)(i - 256) / 1024.0);
+
+    // --- q prep (att_qnorm_scale + att_qrot)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int v = wave + u * nw;
+        if (v >= 16) continue;
+        double ssq = 0.0;
+#pragma unroll
+        for (int c = 0; c < KS; ++c) {
+            const int q = lane + 64 * c < hd ? qa[u][c] : 0;
+            ssq += (double)(q * q);
+        }
+        ssq = wave_sum_exact(ssq);
+        float rq = 1.0f;
+        if (A.qk_norm) {
+            const float ss = (float)ssq * (1.0f / 65536.0f);
+            float r = rsqrt_d(ss / (float)hd + 1e-6f);
+            r = fminf(r, 127.0f);
+            rq = floorf(r * 65536.0f + 0.5f) / 65536.0f;
+        }
+        double sq = 0.0;
+#pragma unroll
+        for (int c = 0; c < KS; ++c) {
+            const int i = lane + 64 * c;
+            int jj, ti;
+            bool first;
+            rope_pair(A.rope_half, hd, min(i, hd - 1), jj, ti, first);
+            const float cf = (float)co[u][c] / 4096.0f, sf = (float)sn[u][c] / 4096.0f;
+            float qv = (float)qa[u][c] / 256.0f, b = (float)qb[u][c] / 256.0f;
+            if (A.qk_norm) {
+                qv = (qv * rq) * ((float)na[u][c] / 256.0f);
+                b = (b * rq) * ((float)nb[u][c] / 256.0f);
+            }
+            const float o = first ? (qv * cf) - (b * sf) : (b * sf) + (qv * cf);
+            const bool on = i < hd && v < nq;
+            const int q = on ? q16_round(o * 256.0f) : 0;
+            sq += (double)q;
+            qp[v * HP + i] = (int8_t)(q >> 8);
+            qp[(16 + v) * HP + i] = on ? (int8_t)((q & 255) - 128) : (int8_t)0;
+        }
+        sq = wave_sum_exact(sq);
+        if (lane == 0) cq[v] = KVB == 16 ? (int)sq : 0;
+    }
+    __syncthreads();
+
+    // --- scores (att_score).  q = 256*qh + ql' + 128 and, at a q16 cache, k =
+    // 256*kh + kl' + 128, so q . k = 256 * hi + lo with
+    //   hi = 256*qh.kh + qh.kl' + ql'.kh,  lo = ql'.kl' + 128*(sum k' + sum q)
+    // (sum k' = sum of 256*kh + kl', from products with ones; the even part of
+    // 128*sum q goes to hi, so neither half leaves int32 up to head_dim 256) and at a q8 cache
+    // hi = qh.k, lo = ql'.k + 128*sum k.
+    {
+        const float invsqrt = 1.0f / sqrtf((float)hd);
+        const float unit = KVB == 16 ? 1.0f / 524288.0f : 1.0f / 4096.0f;
+        v4i qh[KS], ql[KS], one[KS];
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            qh[s] = *reinterpret_cast<const v4i*>(qp + li * HP + 64 * s + 16 * lg);
+            ql[s] = *reinterpret_cast<const v4i*>(qp + (16 + li) * HP + 64 * s + 16 * lg);
+            const int o = 64 * s + 16 * lg < hd ? 0x01010101 : 0;
+            one[s] = (v4i){o, o, o, o};
+        }
+        int cqr[4], npr[4];
+        float mx[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            cqr[r] = cq[4 * lg + r];
+            npr[r] = npos_of(4 * lg + r);
+            mx[r] = -32768.0f;
+        }
+        for (int c = wave; c < nch; c += nw) {
+            // the exact sums as floats: one fused multiply-add where both halves
+            // are exact floats, else the 64-bit integer's conversion
+            float d[8], big = 0.0f;
+            int hi[8], lo[8];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                v4i hh = {}, hl = {}, ll = {}, kh1 = {}, kl1 = {}, kh[KS], kl[KS];
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+#pragma unroll
+                    for (int i = 0; i < NL; ++i) asm volatile("" : "+v"(kr[b][s][i]));
+                    const u32x4 x0 = kr[b][s][0], x1 = kr[b][s][NL - 1];
+                    if (KVB == 16) {
+                        const uint32_t x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+                        uint32_t xh[4], xl[4];
+                        planes16(x, xh, xl);
+                        kh[s] = (v4i){(int)xh[0], (int)xh[1], (int)xh[2], (int)xh[3]};
+                        kl[s] = (v4i){(int)(xl[0] ^ 0x80808080u), (int)(xl[1] ^ 0x80808080u), (int)(xl[2] ^ 0x80808080u),
+                                      (int)(xl[3] ^ 0x80808080u)};
+                    } else {
+                        kl[s] = (v4i){(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w};
+                    }
+                }
+                k_load(c + nw, b);  // the bytes are operands now: the next chunk's go out
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    hl = __builtin_amdgcn_mfma_i32_16x16x64_i8(qh[s], kl[s], hl, 0, 0, 0);
+                    ll = __builtin_amdgcn_mfma_i32_16x16x64_i8(ql[s], kl[s], ll, 0, 0, 0);
+                    kl1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(one[s], kl[s], kl1, 0, 0, 0);
+                    if (KVB == 16) {
+                        hh = __builtin_amdgcn_mfma_i32_16x16x64_i8(qh[s], kh[s], hh, 0, 0, 0);
+                        kh1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(one[s], kh[s], kh1, 0, 0, 0);
+                        hl = __builtin_amdgcn_mfma_i32_16x16x64_i8(ql[s], kh[s], hl, 0, 0, 0);
+                    }
+                }
+                const int sk = 128 * (KVB == 16 ? 256 * kh1[0] + kl1[0] : kl1[0]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    hi[4 * b + r] = KVB == 16 ? 256 * hh[r] + hl[r] + (cqr[r] >> 1) : hl[r];
+                    lo[4 * b + r] = ll[r] + sk + 128 * (cqr[r] & 1);
+                    const float fh = (float)hi[4 * b + r], fl = (float)lo[4 * b + r];
+                    big = fmaxf(big, fmaxf(fabsf(fh), fabsf(fl)));
+                    d[4 * b + r] = __builtin_fmaf(fh, 256.0f, fl);
+                }
+            }
+            if (__any(big >= 16777216.0f)) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k) d[k] = (float)(256ll * hi[k] + lo[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int r = k & 3, t = c * kChunk + 16 * (k >> 2) + li;
+                const float sc = d[k] * unit;
+                const float f = __builtin_amdgcn_fmed3f(floorf((sc * invsqrt) * 1024.0f + 0.5f), -32768.0f, 32767.0f);
+                F[(4 * lg + r) * g.fstride + c * (kChunk + 1) + 16 * (k >> 2) + li] = f;
+                mx[r] = fmaxf(mx[r], t < npr[r] ? f : -32768.0f);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) mx[r] = fmaxf(mx[r], __shfl_xor(mx[r], o, 64));
+            if (li == 0) wmax[wave * 16 + 4 * lg + r] = mx[r];
+        }
+    }
+    __syncthreads();
+
+    // --- weighted V (att_v): a wave takes 16 elements of every query vector and
+    // every second pair of chunks (two sets of waves share an element tile).
+    // Lane: query vector / element li, position 4*s + lg.  The first pair's
+    // values load during the stats.
+    const int ne = hd / 16, set = wave / ne, et = wave - set * ne;
+    const bool act = set < 2;  // (a head of few elements leaves waves without one)
+    const __amdgpu_buffer_rsrc_t vrs = rows_rsrc(vhead, npmax * A.pstride);
+    const int voff = lg * A.pstride + (16 * et + li) * NL;
+    int vr[16];
+    auto v_load = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int off = voff + ((c + (i & 1)) * kChunk + 4 * (i >> 1)) * A.pstride;
+            vr[i] = KVB == 16 ? (int)(int16_t)__builtin_amdgcn_raw_buffer_load_b16(vrs, off, 0, 0)
+                              : (int)(int8_t)__builtin_amdgcn_raw_buffer_load_b8(vrs, off, 0, 0);
+        }
+    };
+    if (act) v_load(2 * set);
+
+    // --- stats (att_stats): the exponentials (+0.0 past each query vector's
+    // context), chunk sums in position order
+    for (int v = wave; v < nq; v += nw) {
+        const int npos = npos_of(v);
+        float m = -32768.0f;
+        for (int w = 0; w < nw; ++w) m = fmaxf(m, wmax[w * 16 + v]);
+        float* Fv = F + v * g.fstride + fidx(lane);  // position t = lane + 64u at + 66u
+        const int ulast = (nch * kChunk - 1) >> 6;
+        for (int u0 = 0; u0 <= ulast; u0 += 4) {
+            float x[4];
+            double ea[4], eb[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] = Fv[66 * min(u0 + u, ulast)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = lane + 64 * (u0 + u) < npos ? (int)(m - x[u]) : 0;
+                ea[u] = tab[k >> 8];
+                eb[u] = tab[256 + (k & 255)];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int t = lane + 64 * (u0 + u);
+                if (t < nch * kChunk) Fv[66 * (u0 + u)] = t < npos ? (float)(ea[u] * eb[u]) : 0.0f;
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < nq * nch; i += 64 * nw) {
+        const int v = i / nch, c = i - v * nch;
+        const float* Fc = F + v * g.fstride + fidx(c * kChunk);
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) s += (double)Fc[k];
+        cs[i] = s;
+    }
+    __syncthreads();
+    float iv = 0.0f;  // 1/sum of query vector li on its grid
+    {
+        // (read unconditionally: under a test each read would be waited for by itself)
+        const double* row = cs + min(li, nq - 1) * nch;
+        double sum = 0.0;
+        for (int c0 = 0; c0 < nch; c0 += 8) {
+            double t[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) t[k] = row[min(c0 + k, nch - 1)];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) sum += c0 + k < nch ? t[k] : 0.0;
+        }
+        const float fs = (float)sum;
+        float qs = floorf(fs * 32.0f + 0.5f);
+        qs = fminf(fmaxf(qs, -32768.0f), 32767.0f);
+        const float sd = qs / 32.0f;
+        iv = sd > 0.0f ? 1.0f / sd : 0.0f;
+    }
+    v4d tot = {0.0, 0.0, 0.0, 0.0};
+    v4d* const X = reinterpret_cast<v4d*>(smem + g.o_x);  // [2][ne][2][64]: the second set's chunk sums
+    const float* Fq = F + li * g.fstride + lg;
+    for (int c0 = 0, rd = 0; c0 < nch; c0 += 4, rd ^= 1) {
+        v4d* const Xr = X + ((rd * ne + et) * 2) * 64 + lane;
+        if (act) {
+            const int c = c0 + 2 * set;
+            int v[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                v[i] = vr[i];
+                asm volatile("" : "+v"(v[i]));
+            }
+            v_load(c + 4);
+            const float* f0 = Fq + min(c, nch - 1) * (kChunk + 1);
+            const float* f1 = Fq + min(c + 1, nch - 1) * (kChunk + 1);
+            v4d acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {  // positions 4*s .. of chunks c and c + 1
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)(f0[4 * s] * iv), (double)v[2 * s], acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)(f1[4 * s] * iv), (double)v[2 * s + 1], acc[1], 0, 0, 0);
+            }
+            // chunk sums in chunk order (a chunk past the end adds nothing)
+            if (set == 0) {
+                tot += acc[0];
+                if (c + 1 < nch) tot += acc[1];
+            } else {
+                Xr[0] = acc[0];
+                Xr[64] = acc[1];
+            }
+        }
+        lds_barrier();
+        if (set == 0) {
+            if (c0 + 2 < nch) tot += Xr[0];
+            if (c0 + 3 < nch) tot += Xr[64];
+        }
+    }
+    if (set) return;
+    const double vunit_d = KVB == 16 ? 1.0 / 2048.0 : 1.0 / 16.0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int v = 4 * r + lg, j = v / hs;
+        if (v < nq)
+            g.out[(size_t)(rbase + j) * A.dim + (h0 + v - j * hs) * hd + 16 * et + li] =
+                (int16_t)q16_round((float)(tot[r] * vunit_d) * 256.0f);
+    }
+}
+
 // LDS carve-up of one workgroup and the lane plan; returns the bytes used.
 // The per-head kernel for A's cache width (A laid out by attn_layout), with the
 // pair plan for a head of at most 32 fields of 32 bits whose cache holds more
@@ -1457,6 +1831,7 @@ size_t attn_layout(AttnDev& A) {
     return off;
 }
 
+int launch_tile(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv, int16_t* out);
 int launch_group(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv, int16_t* out, bool seqs);
 // Sequences in lockstep take the query-block kernel from this many query
 // heads per KV head (every head of a group then reads the K/V rows once).
@@ -1490,6 +1865,10 @@ int launch(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv, int16
     const int16_t* kn = at->kn ? at->kn + (size_t)layer * A.hd : nullptr;
     // a batch of positions, and sequences in lockstep, take the query-block
     // kernel when a block of query vectors fits a workgroup's LDS
+    if (att && !pos_ptr && !seqs && !w && ntok > 1) {
+        const int st = launch_tile(at, layer, pos, ntok, qkv, out);
+        if (st != VGX_ESTATE) return st;
+    }
     if (att && !pos_ptr && ((!seqs && !w && ntok > 1) || (seqs && w && A.group >= kGroupSeqsG))) {
         const int st = launch_group(at, layer, pos, ntok, qkv, out, seqs);
         if (st != VGX_ESTATE) return st;
@@ -1617,6 +1996,62 @@ int launch_group(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv,
     return VGX_OK;
 }
 
+using TileKernel = void (*)(AttnDev, TileArgs);
+TileKernel tile_kernel(int kvb, int ks) {
+    if (ks == 1) return kvb == 16 ? attn_tile_kernel<16, 1> : attn_tile_kernel<8, 1>;
+    return kvb == 16 ? attn_tile_kernel<16, 2> : attn_tile_kernel<8, 2>;
+}
+
+// The tile kernel over rows 0..ntok-1 (positions pos .. pos+ntok-1), as many
+// rows a workgroup as leave about one a CU; VGX_ESTATE when its score rows do
+// not fit the LDS (about 1,500 positions and up), past head_dim 128, and for
+// blocks of few query vectors.
+int launch_tile(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv, int16_t* out) {
+    const AttnDev& A = at->a;
+    if (A.hd > 128) return VGX_ESTATE;
+    TileArgs g{};
+    g.hs = A.group;
+    while (g.hs > 16 && g.hs % 2 == 0) g.hs /= 2;
+    if (g.hs > 16) return VGX_ESTATE;
+    const int nx = A.kv_heads * (A.group / g.hs);
+    const int want = (int)(((long)ntok * nx + at->ctx->num_cu - 1) / at->ctx->num_cu);
+    g.tq = std::max(1, std::min({16 / g.hs, ntok, want}));
+    // Under 8 query vectors a workgroup (a short batch whose KV heads serve few
+    // heads) most of the f64 tile is padding, and the query-block kernel's shorter
+    // phases win: 17 rows at 460, 2 heads of 64 13.3 against 15.9 us, of 96 at a q8
+    // cache 14.7 against 18.4 (33 rows at 100: 10.2 against 12.7); with 8 heads the
+    // tile kernel does, 23.8 -> 15.2.
+    if (g.hs * g.tq < 8) return VGX_ESTATE;
+    g.nby = (ntok + g.tq - 1) / g.tq;
+    if (g.nby > 65535) return VGX_ESTATE;
+    g.nw = std::max(8, A.hd / 8);
+    const int ks = (A.hd + 63) / 64, nch = (pos + ntok + kChunk - 1) / kChunk;
+    g.fstride = (nch * 33 + 63) / 64 * 64 + 4;
+    size_t off = 512 * 8;
+    auto take = [&](size_t bytes) {
+        const size_t o = off;
+        off = (off + bytes + 15) & ~(size_t)15;
+        return (int)o;
+    };
+    g.o_q = take(2 * 16 * 64 * (size_t)ks);
+    g.o_cq = take(16 * 4);
+    g.o_max = take(16 * 4 * (size_t)g.nw);
+    g.o_cs = take(16 * 8 * (size_t)nch);
+    g.o_x = take(2 * 2 * 64 * sizeof(v4d) * (size_t)(A.hd / 16));
+    g.o_f = take(16 * 4 * (size_t)g.fstride + 256);  // (a row's last 64 read past an odd chunk's end)
+    if (off > kLdsMax) return VGX_ESTATE;
+    g.kv = at->kv[layer];
+    g.rtab = at->rtab;
+    g.qn = at->qn ? at->qn + (size_t)layer * A.hd : nullptr;
+    g.qkv = qkv;
+    g.out = out;
+    g.pos0 = pos;
+    g.ntok = ntok;
+    hipLaunchKernelGGL(tile_kernel(A.kv_bits, ks), dim3(nx, g.nby), dim3(64 * g.nw), off, at->ctx->stream, A, g);
+    VGX_LAUNCH_CHECK("tile attention launch");
+    return VGX_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1697,6 +2132,9 @@ int vgx_attn_create_seqs(vgx_ctx* ctx, const vgx_attn_desc* d, int nseq, vgx_att
                                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
                 if (a != hipSuccess) return fail(a, "hipFuncSetAttribute");
             }
+    const hipError_t a2 = hipFuncSetAttribute((const void*)tile_kernel(A.kv_bits, (A.hd + 63) / 64),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
+    if (a2 != hipSuccess) return fail(a2, "hipFuncSetAttribute");
     *out = at;
     return VGX_OK;
 }
