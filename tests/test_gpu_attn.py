@@ -343,6 +343,47 @@ def test_tile_attention_batches(gpu, bits, heads, kvh, hd, seq, batches, rails):
     A.free()
 
 
+# Either side of what the per-head kernel runs at once (256 CUs, one or two
+# workgroups each): short batches and sequences of a few heads take it, the next
+# row or sequence the tile and query-block kernels; head_dim past the tile kernel's.
+# (bits, heads, kv_heads, head_dim, seq, (pos0, rows) ..., rails)
+AT_ONCE = [(16, 8, 1, 64, 320, ((0, 64), (0, 65), (30, 67)), False),
+           (8, 8, 1, 64, 320, ((0, 32), (0, 33), (191, 35)), False),
+           (16, 16, 8, 64, 320, ((0, 32), (0, 33), (257, 33)), False),
+           (8, 32, 1, 32, 160, ((95, 16), (95, 17)), True),
+           (16, 4, 1, 256, 200, ((0, 128), (31, 129)), False),
+           (8, 4, 2, 160, 200, ((0, 64), (31, 129)), False)]
+
+
+@pytest.mark.parametrize("bits,heads,kvh,hd,seq,batches,rails", AT_ONCE)
+def test_batches_around_one_round(gpu, bits, heads, kvh, hd, seq, batches, rails):
+    test_tile_attention_batches(gpu, bits, heads, kvh, hd, seq, batches, rails)
+
+
+@pytest.mark.parametrize("bits,heads,kvh,hd,counts", [(16, 16, 2, 64, (16, 17, 32, 33)), (8, 16, 8, 64, (16, 17, 32)),
+                                                      (16, 8, 4, 96, (32, 34, 64, 65)), (8, 32, 1, 128, (8, 9, 17))])
+def test_sequences_around_one_round(gpu, bits, heads, kvh, hd, counts):
+    rng = np.random.default_rng(heads + hd + bits)
+    seq, nseq = 288, max(counts)
+    A, (c, qnq, knq, rtab), width = _attn_setup(gpu, rng, bits, heads, kvh, hd, seq, nseq=nseq)
+    rows = rng.integers(0, 256, seq * o.kv_row_bytes(c)).astype(np.uint8)
+    for s in range(nseq):
+        A.view(s).write_rows(0, 0, np.roll(rows, 64 * s))
+    for n in counts:
+        for pos in (31, 255, 256, 287):
+            x = np.clip(rng.standard_normal((n, width)) * 700, -32768, 32767).astype(np.int16)
+            X = dev(x)
+            before = A.view(n - 1).read_rows(0, 0, seq).copy()
+            got = A.block_seqs(0, pos, X)
+            # every sequence: one token on its own cache; the last: the oracle
+            for s in range(n):
+                assert torch.equal(A.view(s).decode(0, pos, X[s]), got[s]), (n, pos, s)
+            want = o.attn_block(c, x[n - 1], qnq, knq, rtab, pos, before)
+            assert np.array_equal(got[n - 1].cpu().numpy(), want), (n, pos)
+            assert np.array_equal(A.view(n - 1).read_rows(0, 0, seq), before), (n, pos)
+    A.free()
+
+
 def test_exp_tables_round_as_exp():
     """The tile kernel's exp(-k/1024) = T[k >> 8] * U[k & 255] and the batched
     gate's exp(-g/256) = T'[(g >> 8) + 128] * U'[g & 255], as floats: over every

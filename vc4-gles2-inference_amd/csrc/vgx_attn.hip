@@ -70,6 +70,7 @@ struct vgx_attn {
     int16_t* qn = nullptr;     // [layers][hd] q16
     int16_t* kn = nullptr;
     size_t lds = 0;
+    int per_cu = 1;         // workgroups of the per-head kernel a CU holds
     int nseq = 1;           // sequences whose caches follow one another in each layer
     size_t seq_bytes = 0;   // one sequence's cache of one layer: seq rows
     bool owner = true;      // false for a view of one sequence (shares every buffer)
@@ -1833,6 +1834,7 @@ size_t attn_layout(AttnDev& A) {
 
 int launch_tile(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv, int16_t* out);
 int launch_group(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv, int16_t* out, bool seqs);
+bool heads_at_once(const vgx_attn* at, bool seqs, int pos, int n);
 // Sequences in lockstep take the query-block kernel from this many query
 // heads per KV head (every head of a group then reads the K/V rows once).
 constexpr int kGroupSeqsG = 2;
@@ -1863,13 +1865,16 @@ int launch(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv, int16
     const AttnDev& A = at->a;
     const int16_t* qn = at->qn ? at->qn + (size_t)layer * A.hd : nullptr;
     const int16_t* kn = at->kn ? at->kn + (size_t)layer * A.hd : nullptr;
-    // a batch of positions, and sequences in lockstep, take the query-block
-    // kernel when a block of query vectors fits a workgroup's LDS
-    if (att && !pos_ptr && !seqs && !w && ntok > 1) {
+    // a batch of positions, and sequences in lockstep, past what the per-head
+    // kernel runs at once: the tile kernel (a batch), or the query-block kernel
+    // when a block of query vectors fits a workgroup's LDS
+    const bool blocked = att && !pos_ptr && ((!seqs && !w && ntok > 1) || (seqs && w && A.group >= kGroupSeqsG)) &&
+                         !heads_at_once(at, seqs, pos, ntok);
+    if (blocked && !seqs) {
         const int st = launch_tile(at, layer, pos, ntok, qkv, out);
         if (st != VGX_ESTATE) return st;
     }
-    if (att && !pos_ptr && ((!seqs && !w && ntok > 1) || (seqs && w && A.group >= kGroupSeqsG))) {
+    if (blocked) {
         const int st = launch_group(at, layer, pos, ntok, qkv, out, seqs);
         if (st != VGX_ESTATE) return st;
     }
@@ -1953,6 +1958,32 @@ size_t group_plan(const AttnDev& A, bool seqs, int pos0, int n, int num_cu, Grou
     g.hs = hs;
     g.tq = tq;
     return lds;
+}
+
+// Whether n rows go to the per-head kernel, a workgroup a (row, head).  While
+// the chip holds all of them at once the launch takes about what one token
+// takes: each workgroup runs its whole context with eight waves, where a
+// workgroup of the other kernels runs several query vectors one phase after
+// another and reads K and V no sooner.  us, per-head against the better of the
+// others: 17 rows at 460 with 8 heads of 96, q16 10.3 / 17.2, q8 8.4 / 14.7; 17
+// rows of 16 heads of 64 at 460 (two workgroups on some CUs) 10.9 / 13.3; 32 of
+// them at 500 12.7 / 15.8, at 4,000 50.8 / 64.8.  With one more round it is no
+// longer so (33 rows at 0 9.8 / 9.0; a q8 cache with heads of 64, whose instance
+// has one workgroup a CU, 17 rows at 300 13.1 / 10.5).
+//
+// Sequences each have a cache of their own, so two workgroups on a CU share its
+// bandwidth: they keep to it as long as what the launch reads comes to at most
+// 128 KB a CU (32 sequences of 16 heads of 64: at 130 8.3 / 10.0, at 255 9.3 /
+// 10.5, at 270 11.5 / 11.8, at 320 13.7 / 12.1), or the query-block kernel, one
+// workgroup a CU, would need a second round (17 sequences at 255 8.9 / 18.0).
+bool heads_at_once(const vgx_attn* at, bool seqs, int pos, int n) {
+    const AttnDev& A = at->a;
+    const int num_cu = at->ctx->num_cu;
+    const long blocks = (long)A.heads * n;
+    if (blocks > (long)num_cu * at->per_cu) return false;
+    if (!seqs || blocks <= num_cu || blocks * (pos + 1) * 2 * A.pstride <= (long)num_cu * (128 << 10)) return true;
+    GroupArgs g{};
+    return !group_plan(A, true, pos, n, num_cu, g) || (long)A.kv_heads * (A.group / g.hs) * n > num_cu;
 }
 
 using GroupKernel = void (*)(AttnDev, GroupArgs);
@@ -2125,6 +2156,9 @@ int vgx_attn_create_seqs(vgx_ctx* ctx, const vgx_attn_desc* d, int nseq, vgx_att
     const hipError_t a1 = hipFuncSetAttribute((const void*)attn_kernel_for(A),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
     if (a1 != hipSuccess) return fail(a1, "hipFuncSetAttribute");
+    const hipError_t ao = hipOccupancyMaxActiveBlocksPerMultiprocessor(&at->per_cu, attn_kernel_for(A), kThreads, 0);
+    if (ao != hipSuccess) return fail(ao, "attention occupancy");
+    at->per_cu = std::max(1, std::min(at->per_cu, (int)(kLdsMax / at->lds)));
     for (int kvb : {16, 8})
         for (int ve : {1, 2})
             for (int qg : {2, 4}) {
