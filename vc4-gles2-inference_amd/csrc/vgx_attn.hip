@@ -1575,63 +1575,70 @@ __global__ void __launch_bounds__(512 * KS, 4) attn_tile_kernel(const AttnDev A,
             npr[r] = npos_of(4 * lg + r);
             mx[r] = -32768.0f;
         }
+        // 16-position blocks whose sums are held at once: both of a chunk's, but for
+        // the widest rows, where they would not fit the 128 registers of a lane
+        constexpr int NB = KVB == 16 && KS == 2 ? 1 : 2;
         for (int c = wave; c < nch; c += nw) {
-            // the exact sums as floats: one fused multiply-add where both halves
-            // are exact floats, else the 64-bit integer's conversion
-            float d[8], big = 0.0f;
-            int hi[8], lo[8];
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                v4i hh = {}, hl = {}, ll = {}, kh1 = {}, kl1 = {}, kh[KS], kl[KS];
+            for (int b0 = 0; b0 < 2; b0 += NB) {
+                // the exact sums as floats: one fused multiply-add where both halves
+                // are exact floats, else the 64-bit integer's conversion
+                float d[4 * NB], big = 0.0f;
+                int hi[4 * NB], lo[4 * NB];
 #pragma unroll
-                for (int s = 0; s < KS; ++s) {
+                for (int b = b0; b < b0 + NB; ++b) {
+                    const int k0 = 4 * (b - b0);
+                    v4i hh = {}, hl = {}, ll = {}, kh1 = {}, kl1 = {}, kh[KS], kl[KS];
 #pragma unroll
-                    for (int i = 0; i < NL; ++i) asm volatile("" : "+v"(kr[b][s][i]));
-                    const u32x4 x0 = kr[b][s][0], x1 = kr[b][s][NL - 1];
-                    if (KVB == 16) {
-                        const uint32_t x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-                        uint32_t xh[4], xl[4];
-                        planes16(x, xh, xl);
-                        kh[s] = (v4i){(int)xh[0], (int)xh[1], (int)xh[2], (int)xh[3]};
-                        kl[s] = (v4i){(int)(xl[0] ^ 0x80808080u), (int)(xl[1] ^ 0x80808080u), (int)(xl[2] ^ 0x80808080u),
-                                      (int)(xl[3] ^ 0x80808080u)};
-                    } else {
-                        kl[s] = (v4i){(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w};
+                    for (int s = 0; s < KS; ++s) {
+#pragma unroll
+                        for (int i = 0; i < NL; ++i) asm volatile("" : "+v"(kr[b][s][i]));
+                        const u32x4 x0 = kr[b][s][0], x1 = kr[b][s][NL - 1];
+                        if (KVB == 16) {
+                            const uint32_t x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+                            uint32_t xh[4], xl[4];
+                            planes16(x, xh, xl);
+                            kh[s] = (v4i){(int)xh[0], (int)xh[1], (int)xh[2], (int)xh[3]};
+                            kl[s] = (v4i){(int)(xl[0] ^ 0x80808080u), (int)(xl[1] ^ 0x80808080u), (int)(xl[2] ^ 0x80808080u),
+                                          (int)(xl[3] ^ 0x80808080u)};
+                        } else {
+                            kl[s] = (v4i){(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w};
+                        }
+                    }
+                    k_load(c + nw, b);  // the bytes are operands now: the next chunk's go out
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) {
+                        hl = __builtin_amdgcn_mfma_i32_16x16x64_i8(qh[s], kl[s], hl, 0, 0, 0);
+                        ll = __builtin_amdgcn_mfma_i32_16x16x64_i8(ql[s], kl[s], ll, 0, 0, 0);
+                        kl1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(one[s], kl[s], kl1, 0, 0, 0);
+                        if (KVB == 16) {
+                            hh = __builtin_amdgcn_mfma_i32_16x16x64_i8(qh[s], kh[s], hh, 0, 0, 0);
+                            kh1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(one[s], kh[s], kh1, 0, 0, 0);
+                            hl = __builtin_amdgcn_mfma_i32_16x16x64_i8(ql[s], kh[s], hl, 0, 0, 0);
+                        }
+                    }
+                    const int sk = 128 * (KVB == 16 ? 256 * kh1[0] + kl1[0] : kl1[0]);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        hi[k0 + r] = KVB == 16 ? 256 * hh[r] + hl[r] + (cqr[r] >> 1) : hl[r];
+                        lo[k0 + r] = ll[r] + sk + 128 * (cqr[r] & 1);
+                        const float fh = (float)hi[k0 + r], fl = (float)lo[k0 + r];
+                        big = fmaxf(big, fmaxf(fabsf(fh), fabsf(fl)));
+                        d[k0 + r] = __builtin_fmaf(fh, 256.0f, fl);
                     }
                 }
-                k_load(c + nw, b);  // the bytes are operands now: the next chunk's go out
+                if (__any(big >= 16777216.0f)) {
 #pragma unroll
-                for (int s = 0; s < KS; ++s) {
-                    hl = __builtin_amdgcn_mfma_i32_16x16x64_i8(qh[s], kl[s], hl, 0, 0, 0);
-                    ll = __builtin_amdgcn_mfma_i32_16x16x64_i8(ql[s], kl[s], ll, 0, 0, 0);
-                    kl1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(one[s], kl[s], kl1, 0, 0, 0);
-                    if (KVB == 16) {
-                        hh = __builtin_amdgcn_mfma_i32_16x16x64_i8(qh[s], kh[s], hh, 0, 0, 0);
-                        kh1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(one[s], kh[s], kh1, 0, 0, 0);
-                        hl = __builtin_amdgcn_mfma_i32_16x16x64_i8(ql[s], kh[s], hl, 0, 0, 0);
-                    }
+                    for (int k = 0; k < 4 * NB; ++k) d[k] = (float)(256ll * hi[k] + lo[k]);
                 }
-                const int sk = 128 * (KVB == 16 ? 256 * kh1[0] + kl1[0] : kl1[0]);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    hi[4 * b + r] = KVB == 16 ? 256 * hh[r] + hl[r] + (cqr[r] >> 1) : hl[r];
-                    lo[4 * b + r] = ll[r] + sk + 128 * (cqr[r] & 1);
-                    const float fh = (float)hi[4 * b + r], fl = (float)lo[4 * b + r];
-                    big = fmaxf(big, fmaxf(fabsf(fh), fabsf(fl)));
-                    d[4 * b + r] = __builtin_fmaf(fh, 256.0f, fl);
+                for (int k = 0; k < 4 * NB; ++k) {
+                    const int r = k & 3, p = 16 * (b0 + (k >> 2)) + li, t = c * kChunk + p;
+                    const float sc = d[k] * unit;
+                    const float f = __builtin_amdgcn_fmed3f(floorf((sc * invsqrt) * 1024.0f + 0.5f), -32768.0f, 32767.0f);
+                    F[(4 * lg + r) * g.fstride + c * (kChunk + 1) + p] = f;
+                    mx[r] = fmaxf(mx[r], t < npr[r] ? f : -32768.0f);
                 }
-            }
-            if (__any(big >= 16777216.0f)) {
-#pragma unroll
-                for (int k = 0; k < 8; ++k) d[k] = (float)(256ll * hi[k] + lo[k]);
-            }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int r = k & 3, t = c * kChunk + 16 * (k >> 2) + li;
-                const float sc = d[k] * unit;
-                const float f = __builtin_amdgcn_fmed3f(floorf((sc * invsqrt) * 1024.0f + 0.5f), -32768.0f, 32767.0f);
-                F[(4 * lg + r) * g.fstride + c * (kChunk + 1) + 16 * (k >> 2) + li] = f;
-                mx[r] = fmaxf(mx[r], t < npr[r] ? f : -32768.0f);
             }
         }
 #pragma unroll
