@@ -285,7 +285,7 @@ def test_query_block_sequences(gpu, bits, heads, kvh, hd, seq):
     A.free()
 
 
-# The tile kernel (8 or more query vectors a workgroup): query vectors of 8, 16,
+# The tile kernel (4 or 5 query vectors a workgroup and up): query vectors of 8, 16,
 # 32, 3, 1 and 2 heads a KV head, head_dim of one to eight element tiles (one and
 # two 64-wide key steps, the second padded), batches that end inside a block,
 # contexts around a chunk and a round of four chunks, cached rows at the rails.
@@ -345,14 +345,17 @@ def test_tile_attention_batches(gpu, bits, heads, kvh, hd, seq, batches, rails):
 
 # Either side of what the per-head kernel runs at once (256 CUs, one or two
 # workgroups each): short batches and sequences of a few heads take it, the next
-# row or sequence the tile and query-block kernels; head_dim past the tile kernel's.
+# row or sequence the tile and query-block kernels, each side of the query vectors a
+# workgroup that the tile kernel asks for; head_dim past the tile kernel's.
 # (bits, heads, kv_heads, head_dim, seq, (pos0, rows) ..., rails)
 AT_ONCE = [(16, 8, 1, 64, 320, ((0, 64), (0, 65), (30, 67)), False),
            (8, 8, 1, 64, 320, ((0, 32), (0, 33), (191, 35)), False),
            (16, 16, 8, 64, 320, ((0, 32), (0, 33), (257, 33)), False),
            (8, 32, 1, 32, 160, ((95, 16), (95, 17)), True),
            (16, 4, 1, 256, 200, ((0, 128), (31, 129)), False),
-           (8, 4, 2, 160, 200, ((0, 64), (31, 129)), False)]
+           (8, 4, 2, 160, 200, ((0, 64), (31, 129)), False),
+           (8, 16, 8, 64, 320, ((0, 33), (257, 40), (200, 65)), False),
+           (16, 8, 8, 96, 200, ((0, 65), (100, 70), (60, 129)), False)]
 
 
 @pytest.mark.parametrize("bits,heads,kvh,hd,seq,batches,rails", AT_ONCE)

@@ -2054,12 +2054,13 @@ int launch_tile(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv, 
     const int nx = A.kv_heads * (A.group / g.hs);
     const int want = (int)(((long)ntok * nx + at->ctx->num_cu - 1) / at->ctx->num_cu);
     g.tq = std::max(1, std::min({16 / g.hs, ntok, want}));
-    // Under 8 query vectors a workgroup (a short batch whose KV heads serve few
-    // heads) most of the f64 tile is padding, and the query-block kernel's shorter
-    // phases win: 17 rows at 460, 2 heads of 64 13.3 against 15.9 us, of 96 at a q8
-    // cache 14.7 against 18.4 (33 rows at 100: 10.2 against 12.7); with 8 heads the
-    // tile kernel does, 23.8 -> 15.2.
-    if (g.hs * g.tq < 8) return VGX_ESTATE;
+    // With few query vectors a workgroup (a batch of few rows whose KV heads serve
+    // few heads) most of the f64 tile is padding, and the query-block kernel's shorter
+    // phases win.  It runs one V pass up to 4, two up to 8; us at position 500, it
+    // against this kernel: heads of 64, q8 cache, 2 vectors 13.1 / 17.1, 4 16.8 / 17.4,
+    // 6 22.2 / 17.7; q16 4 20.2 / 18.1, 6 26.7 / 18.4; heads of 96, q8 4 21.2 / 21.5, 6
+    // 33.8 / 24.3; q16 4 25.3 / 22.8, 6 38.6 / 25.8.
+    if (g.hs * g.tq < (A.kv_bits == 16 ? 4 : 5)) return VGX_ESTATE;
     g.nby = (ntok + g.tq - 1) / g.tq;
     if (g.nby > 65535) return VGX_ESTATE;
     g.nw = std::max(8, A.hd / 8);
