@@ -667,7 +667,8 @@ bool workspace(vgx_ctx* ctx, size_t bytes, long long** out) {
     return true;
 }
 
-// Waves per workgroup: 4 when the launch has at least one tile per CU (two
+// Waves per workgroup (measured when every batched launch ran here; now the
+// RMSNorm-fused ones and q4 of one token tile): 4 when the launch has at least one tile per CU (two
 // 4-wave workgroups fit a CU's registers where one 8-wave workgroup does, so
 // up to two tiles a CU run in one round: the 256-token qkv, 384 tiles, took
 // 0.8% less of MiniMind3's 256-token q4 prefill than with 8 waves in two rounds); otherwise (a

@@ -414,7 +414,7 @@ struct vgx_engine {
                       : vgx_gemm(ctx, in_mat, n, bxn, nullptr, bqkv);
             if (st) return st;
             if (is_conv(l)) {
-                // the conv over the batch walks its positions in order
+                // the conv over the whole batch
                 if ((st = vgx_conv_step(conv, l, n, bqkv, batt))) return st;
                 if ((st = vgx_gemm(ctx, ly.conv_out, n, batt, bh, bx1))) return st;
             } else {
