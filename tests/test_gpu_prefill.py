@@ -164,6 +164,45 @@ def test_gemm_sums_past_24_bits(gpu, kind):
             assert np.array_equal(got[t], want), (split, t)
 
 
+# Exact sums of up to 2^49, which the widest q4 rows reach at the rails: below and
+# above 2^47 and 2^48 in either sign, in launches where some rows do and where all
+# do, with every epilogue (one token tile and several).
+@pytest.mark.parametrize("cols", [4096, 8192, 16384, 32768])
+@pytest.mark.parametrize("ntok,every", [(70, False), (64, True), (20, True)])
+def test_gemm_q4_sums_at_the_rails(gpu, cols, ntok, every):
+    from vgx import mmcf
+    rng = np.random.default_rng(cols + ntok)
+    rows, groups = 64, cols // 32
+
+    def matrix():
+        nib = np.full((rows, cols // 2), 0xFF, np.uint8)
+        s16 = np.full((rows, groups), 32767, np.int16)
+        m16 = np.full((rows, groups), 32767, np.int16)
+        s16[1::4] = m16[1::4] = -32768
+        if not every:
+            nib[2::4] = rng.integers(0, 256, nib[2::4].shape)
+            s16[3::4] = rng.integers(-300, 300, s16[3::4].shape)
+        # the largest sum, 2^34 a column, is 32,000 in output units
+        return mmcf.Matrix("q4", rows, cols, nib.ravel(), 32000.0 / (2.0 ** 34 * cols), s16=s16.ravel(), m16=m16.ravel())
+
+    m, m3 = matrix(), matrix()
+    W, W3 = gpu.upload(m), gpu.upload(m3)
+    x = np.full((ntok, cols), 32767, np.int16)
+    x[1::2] = -32768
+    if not every:
+        x[2::3] = x_rows(rng, len(x[2::3]), cols)
+    res = x_rows(rng, ntok, rows)
+    half = cols // 2
+    got, got_s = host(gpu.gemm(W, dev(x), res=dev(res))), host(gpu.gemm_add_split(W, half, dev(x), dev(res)))
+    gate = host(gpu.ffn_gate_batch(W, W3, dev(x), 1))
+    a, b = m.slice_cols(0, half), m.slice_cols(half, cols)
+    for t in range(ntok):
+        v = oracle_rowval(m, x[t])
+        assert np.array_equal(got[t], o.store(v, res[t])), t
+        assert np.array_equal(got_s[t], o.store(oracle_rowval(b, x[t, half:]), o.store(oracle_rowval(a, x[t, :half]), res[t]))), t
+        assert np.array_equal(gate[t], o.gate(v, oracle_rowval(m3, x[t]), 1)), t
+
+
 @pytest.mark.parametrize("chunk", [32, 8192, 65536])
 def test_gate_every_input(gpu, chunk):
     """The batched gate's table exponential and refined quotient at every one

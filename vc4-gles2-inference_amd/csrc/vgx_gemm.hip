@@ -187,8 +187,11 @@ __device__ __forceinline__ float gate_value_tab(float v1, float v3, float f, con
     return r * ((float)q16_med(v3) * 0.00390625f) * f;
 }
 
-// An output's exact sum: 256 * hi + lo (q8, t3; |hi|, |lo| < 2^31 for K <=
-// 32768), or the int64 (q4).
+// The widest matrix that is uploaded; the bounds of the sums below rest on it.
+constexpr int kMaxCols = 32768;
+
+// An output's exact sum: 256 * hi + lo (q8, t3; |hi|, |lo| <= 2^30 at kMaxCols
+// columns), or the int64 (q4).
 template <int KIND>
 struct Sum {
     int hi, lo;
@@ -207,10 +210,13 @@ struct Sum<VGX_Q4> {
     long long v;
     __device__ __forceinline__ void add(const Sum& o) { v += o.v; }
     __device__ __forceinline__ float slow() const { return (float)v; }
+    // The high part is an int for every |v| < 2^55: no row reaches past 2^49
+    // (kMaxCols columns of 2^15 * 2^19), and from 2^48 on it is no exact float,
+    // which mx shows.
     __device__ __forceinline__ float fast(float& mx) const {
-        const float fh = (float)(int)(v >> 16), fl = (float)(int)(v & 0xFFFF);  // (|v| < 2^47)
+        const float fh = (float)(int)(v >> 24), fl = (float)(int)(v & 0xFFFFFF);
         mx = fmaxf(mx, fabsf(fh));
-        return __builtin_fmaf(fh, 65536.0f, fl);
+        return __builtin_fmaf(fh, 16777216.0f, fl);
     }
 };
 
@@ -677,8 +683,8 @@ hipError_t vgx_gemm_tile_init(int num_cu) {
 }
 
 int vgx_gemm_tile_launch(const GemmLaunch& L, int epi, int num_cu, hipStream_t s) {
-    // 32-bit sums (|lo| <= 2^15 * K) and 32-bit offsets within a workgroup's rows
-    if (L.cols > 65535 || L.M.rows > (1 << 22)) return VGX_ESTATE;
+    // the sums' ranges, and 32-bit offsets within a workgroup's rows
+    if (L.cols > kMaxCols || L.M.rows > (1 << 22)) return VGX_ESTATE;
     const int kind = L.M.kind;
     // A q4 launch of one token tile: dequantised into three planes for 32
     // tokens only, a weight costs more here than its share of the group sums
