@@ -83,7 +83,7 @@ int vgx_ctx_create(int device, vgx_ctx** out) {
     c->device = device;
     c->num_cu = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
     c->scratch_keys = keys;
-    hipError_t e = vgx_gemm_tile_init(c->num_cu);
+    hipError_t e = vgx_gemm_tile_init();
     if (e == hipSuccess) e = hipStreamCreate(&c->own);
     if (e != hipSuccess) {
         delete c;

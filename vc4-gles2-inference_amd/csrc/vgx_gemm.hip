@@ -623,58 +623,89 @@ TilePlan plan() {
 // these launches are a few microseconds, set by the chain of one k tile (LDS
 // write, barrier, LDS read, matrix cores) and by the epilogue of a wave, so
 // many short waves beat few wide ones until a launch has several tiles a CU.
-// `tiles` is the launch's count of 32 x 32 output tiles.  Measured, us a call,
-// against the one-token-tile kernel of vgx_prefill.hip that all of these took
-// (tokens x rows x columns):
-//   up to a tile a CU, K over 8 one-wave groups (no barrier in the loop):
-//     q8 512 x 768 x 768 residual 6.9 -> 5.9, q8 256 x 768 x 768 4.9 -> 4.5;
-//     two-half residual q8 256 x 768 x 2432 9.4 -> 6.0, 256 x 1024 x 4608
-//     15.3 -> 9.1, q4 14.5 -> 10.4 and 27.5 -> 16.4, t3 32 x 1024 x 4096 9.9
-//     (two launches) -> 8.6
-//   up to 2.2 tiles a CU, four groups of two waves on 64 tokens:
-//     q8 256 x 1536 x 768 6.6 -> 5.8, q4 9.2 -> 7.9 (8 one-wave groups: 6.0, 17.6)
-//   more, two groups of 2 x 2 waves: q8 512 x 2048 x 1024 10.9 -> 7.5, q4 17.3 -> 11.5
-//   gate, up to a tile a CU: q8 32 x 2432 x 768 7.5 -> 5.6; to 3.5 tiles a
-//     CU: q8 256 x 2432 x 768 13.5 -> 9.1, q4 20.5 -> 13.7 (two token tiles a wave:
-//     three planes of weights a step want more tokens each); beyond, no K groups:
-//     q8 256 x 4608 x 1024 25.4 -> 13.3; past 6 tiles a CU W1 and W3 in one wave:
-//     512 x 4608 x 1024 40.5 -> 20.2 (22.7 with the plan before), t3 512 x 4096 x
-//     1024 36.4 -> 18.3, q4 66.2 -> 40.9 (the plan before)
+//   store  0: 32 x 32 outputs a workgroup, K over 8 one-wave groups (no barrier
+//             in the loop); 1: 64 x 32, four groups of two waves; 2: 64 x 64, two
+//             groups of 2 x 2 waves
+//   split  0: 32 x 32, 8 one-wave groups; 1: 64 x 32, the same
+//   gate   0: 32 x 32, four groups (W1 and W3 in a wave each); 1: 64 x 32, two
+//             groups; 2 (q4): 128 x 32, two groups (three planes of weights a step
+//             want more tokens each); 3: 64 x 32, no K groups; 4 (q8, t3): 64 x 64,
+//             W1 and W3 in one wave
+// us a call, the one-token-tile kernel of vgx_prefill.hip before and the plan after
+// (tokens x rows x columns): store 0 q8 512 x 768 x 768 6.9 -> 5.9; 1 q8 256 x 1536
+// x 768 6.6 -> 5.8, q4 9.2 -> 7.9; 2 q8 512 x 2048 x 1024 10.9 -> 7.5, q4 17.3 ->
+// 11.5; split 0 q8 256 x 768 x 2432 9.4 -> 6.0, q4 14.5 -> 10.4; gate 0 q8 32 x
+// 2432 x 768 7.5 -> 5.6; 1 q8 256 x 2432 x 768 13.5 -> 9.1; 2 q4 the same 20.5 ->
+// 13.7; 3 q8 256 x 4608 x 1024 25.4 -> 13.3; 4 q8 512 x 4608 x 1024 40.5 -> 20.2.
 template <int KIND>
-TilePlan pick_plan(int epi, long tiles, int num_cu) {
+TilePlan plan_of(int epi, int i) {
     constexpr bool q4 = KIND == VGX_Q4;
-    const bool few = tiles <= num_cu;
-    if (epi == BEPI_SPLIT)
-        return few ? plan<KIND, BEPI_SPLIT, 1, 1, 1, 1, 8, 2>() : plan<KIND, BEPI_SPLIT, 2, 1, 1, 1, 8, 2>();
-    if (epi == BEPI_STORE) {
-        if (few) return plan<KIND, BEPI_STORE, 1, 1, 1, 1, 8, 2>();
-        if (tiles * 5 <= 11L * num_cu) return plan<KIND, BEPI_STORE, 1, 1, 2, 1, 4, 2>();
-        return plan<KIND, BEPI_STORE, 1, 1, 2, 2, 2, 2>();
+    if (epi == BEPI_STORE) switch (i) {
+        case 0: return plan<KIND, BEPI_STORE, 1, 1, 1, 1, 8, 2>();
+        case 1: return plan<KIND, BEPI_STORE, 1, 1, 2, 1, 4, 2>();
+        case 2: return plan<KIND, BEPI_STORE, 1, 1, 2, 2, 2, 2>();
     }
-    if (few) return plan<KIND, BEPI_GATE, 1, 1, 1, 2, 4, 2>();
-    if (tiles * 2 <= 7L * num_cu) {
-        if (q4 && tiles * 4 > 7L * num_cu) return plan<KIND, BEPI_GATE, 2, 1, 2, 2, 2, 2>();
-        return plan<KIND, BEPI_GATE, 1, 1, 2, 2, 2, 2>();
+    if (epi == BEPI_SPLIT) switch (i) {
+        case 0: return plan<KIND, BEPI_SPLIT, 1, 1, 1, 1, 8, 2>();
+        case 1: return plan<KIND, BEPI_SPLIT, 2, 1, 1, 1, 8, 2>();
     }
-    if (!q4 && tiles > 6L * num_cu) return plan<KIND, BEPI_GATE, 1, q4 ? 1 : 2, 2, 2, 1, 2>();
-    return plan<KIND, BEPI_GATE, 1, 1, 2, 2, 1, 2>();
+    if (epi == BEPI_GATE) switch (i) {
+        case 0: return plan<KIND, BEPI_GATE, 1, 1, 1, 2, 4, 2>();
+        case 1: return plan<KIND, BEPI_GATE, 1, 1, 2, 2, 2, 2>();
+        case 2: if constexpr (q4) return plan<KIND, BEPI_GATE, 2, 1, 2, 2, 2, 2>(); else break;
+        case 3: return plan<KIND, BEPI_GATE, 1, 1, 2, 2, 1, 2>();
+        case 4: if constexpr (!q4) return plan<KIND, BEPI_GATE, 1, 2, 2, 2, 1, 2>(); else break;
+    }
+    return TilePlan{};
 }
 
-TilePlan pick_plan(int kind, int epi, long tiles, int num_cu) {
-    return kind == VGX_Q8   ? pick_plan<VGX_Q8>(epi, tiles, num_cu)
-           : kind == VGX_Q4 ? pick_plan<VGX_Q4>(epi, tiles, num_cu)
-                            : pick_plan<VGX_T3>(epi, tiles, num_cu);
+TilePlan plan_of(int kind, int epi, int i) {
+    return kind == VGX_Q8 ? plan_of<VGX_Q8>(epi, i) : kind == VGX_Q4 ? plan_of<VGX_Q4>(epi, i) : plan_of<VGX_T3>(epi, i);
+}
+
+// Which plan: the one whose workgroups fill the chip's rounds best.  A CU runs one
+// workgroup of 64 x 32 (its operands take half the LDS and a little more) or, for
+// q8 and t3, two of 32 x 32, and a second round costs about as much as the first,
+// so what decides is each plan's own count of workgroups and not the launch's size
+// alone.  us a call at 1,024 columns, the plan's number before each (q8; q4 after
+// the bar):
+//   96 x 4608 store: 0 6.4, 1 (288 workgroups) 10.9, 2 7.0 | 0 11.9, 1 15.8, 2 10.8
+//   200 x 2432 store: 0 8.6, 1 (304) 11.1, 2 7.3 | 0 16.6, 1 15.7, 2 10.9
+//   256 x 2048 store: 0 6.7, 1 (256) 6.5, 2 7.2 | 0 11.8, 1 8.8, 2 10.8
+//   96 x 4608 gate: 0 8.6, 1 (288) 10.1, 3 10.6, 4 11.2 | 0 19.1, 1 20.9, 2 16.1, 3 17.8
+//   256 x 2048 gate: 0 8.9, 1 (256) 7.5, 3 8.9, 4 11.2 | 0 19.5, 1 11.6, 2 16.3, 3 13.4
+//   64 x 9600 gate: 0 12.0, 1 (300) 10.2, 3 10.6, 4 13.1 | 0 27.6, 1 20.8, 2 (300) 31.1, 3 17.9
+//   200 x 4608 gate: 0 15.1, 1 (576) 14.9, 3 13.0, 4 14.5 | 1 30.2, 2 31.6, 3 24.3
+//   256 x 6400 gate: 3 16.4, 4 14.8
+// and the two-half residual of 2,432 columns, where a plan-1 workgroup takes as long
+// as two rounds of plan 0 (q4, one 32 x 32 workgroup a CU: 1.5 rounds):
+//   96 x 4608: 0 9.6, 1 (2 rounds) 16.1 | 0 18.9, 1 26.6
+//   384 x 2048: 0 14.3, 1 (2) 16.6 | 0 27.9, 1 26.8
+//   512 x 2048: 0 18.4, 1 (2) 17.7 | 0 36.8, 1 27.9
+int pick_plan(int kind, int epi, int rows, int ntok, int num_cu) {
+    const bool q4 = kind == VGX_Q4;
+    auto blocks = [&](int tokens) { return (long)((rows + kTile - 1) / kTile) * ((ntok + tokens - 1) / tokens); };
+    auto rounds = [&](int tokens) { return (blocks(tokens) + num_cu - 1) / num_cu; };
+    const long b32 = blocks(32), b64 = blocks(64);
+    if (b32 <= num_cu) return 0;
+    if (epi == BEPI_SPLIT) return q4 ? 3 * rounds(64) <= 2 * rounds(32) : 2 * rounds(64) <= rounds(32);
+    if (b64 <= num_cu) return 1;
+    if (epi == BEPI_STORE) return !q4 && b32 <= 2L * num_cu ? 0 : 2;
+    if (q4) return blocks(128) <= num_cu ? 2 : 3;
+    if (b32 <= 2L * num_cu) return 0;
+    if (b64 <= 2L * num_cu) return 1;
+    return b32 > 6L * num_cu ? 4 : 3;
 }
 
 }  // namespace
 
 // LDS past 64 KB is granted per kernel, once a context (not on the launch path).
-hipError_t vgx_gemm_tile_init(int num_cu) {
+hipError_t vgx_gemm_tile_init() {
     for (int kind : {VGX_Q8, VGX_Q4, VGX_T3})
         for (int epi : {BEPI_STORE, BEPI_GATE, BEPI_SPLIT})
-            for (long tiles : {1L, 3L * num_cu / 2, 5L * num_cu / 2, 5L * num_cu, 8L * num_cu}) {  // each plan once or more
-                const TilePlan P = pick_plan(kind, epi, tiles, num_cu);
-                if (P.lds <= 64 * 1024) continue;
+            for (int i = 0; i < 5; ++i) {
+                const TilePlan P = plan_of(kind, epi, i);
+                if (P.lds <= 64 * 1024) continue;  // (no such plan: 0)
                 const hipError_t e =
                     hipFuncSetAttribute((const void*)P.fn, hipFuncAttributeMaxDynamicSharedMemorySize, P.lds);
                 if (e != hipSuccess) return e;
@@ -691,8 +722,7 @@ int vgx_gemm_tile_launch(const GemmLaunch& L, int epi, int num_cu, hipStream_t s
     // in the one-tile kernel (32 x 1024 x 4608 two-half residual 14.6 against 11.5 us,
     // 32 x 768 x 768 6.3 against 5.9); not so the gate, whose epilogue is faster (12.1 -> 10.2).
     if (kind == VGX_Q4 && L.ntok <= kTile && epi != BEPI_GATE) return VGX_ESTATE;
-    const long tiles = (long)((L.M.rows + kTile - 1) / kTile) * ((L.ntok + kTile - 1) / kTile);
-    const TilePlan P = pick_plan(kind, epi, tiles, num_cu);
+    const TilePlan P = plan_of(kind, epi, pick_plan(kind, epi, L.M.rows, L.ntok, num_cu));
     const long ntx = (L.M.rows + P.rb - 1) / P.rb, nty = (L.ntok + P.bm - 1) / P.bm;
     const long blocks = (ntx + 7) / 8 * 8 * nty;
     if (blocks > 0x7FFFFFFFL) return VGX_ESTATE;

@@ -156,6 +156,6 @@ struct GemvLaunch {
 
 int vgx_gemv_plan(int kind, int rows, int cols, int num_cu, int* lpr, int* ri, int* rows_per_block);
 int vgx_gemv_launch(const GemvLaunch& L, hipStream_t s);
-hipError_t vgx_gemm_tile_init(int num_cu);  // vgx_gemm.hip, with the device current
+hipError_t vgx_gemm_tile_init();  // vgx_gemm.hip, with the device current
 int vgx_argmax_launch(const int16_t* v, int n, int rows, int* out, hipStream_t s);
 int vgx_dequant_launch(const MatDev& d, float* out, hipStream_t s);
