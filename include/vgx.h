@@ -221,9 +221,10 @@ int vgx_logits_argmax_rms_noalloc(vgx_ctx* ctx, const vgx_group* g, const int16_
  *     qkv and out rows consecutive; the KV rows are written first, then every
  *     position attends to its prefix (att_stage, att_scores_batch,
  *     att_stats_row, att_v_row: engine/src/gpu_attn.cpp:433-532).
- * A q4 vgx_gemm or vgx_gemm_add_split launch of at most 32 tokens whose row
- * tiles leave most CUs idle and whose rows are longer than
- * 32 k-steps (of 32 columns) splits K over up to 8 workgroups
+ * A vgx_gemm, vgx_gemm_add_split or vgx_ffn_gate_batch launch of at most 32
+ * tokens whose row tiles leave most CUs idle and whose rows are long enough for
+ * it to pay (q4: longer than 32 k-steps of 32 columns; q8 and t3: from about 1,500
+ * to 8,000 columns on) splits K over up to 8 workgroups
  * and adds their exact integer sums in a second launch; the sums live in a
  * workspace of the context, sized for every such launch (8 splits x 2 sets x
  * 32 tokens x num_cu/2 tiles of 32 rows, int64: 16 MiB at 256 CUs), allocated

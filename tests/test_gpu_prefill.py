@@ -203,6 +203,58 @@ def test_gemm_q4_sums_at_the_rails(gpu, cols, ntok, every):
         assert np.array_equal(gate[t], o.gate(v, oracle_rowval(m3, x[t]), 1)), t
 
 
+# Each side of the lines between the tile kernel, the one-token-tile kernel and its
+# split pair: long rows over one token tile, more row tiles than CUs, 16 and 17
+# tokens, q4's 24 k-steps, second rounds of a few workgroups, and rows past the tile
+# kernel's limit.  (kinds, rows, cols, tokens)
+ROUTES = [("q8 q4 t3", 96, 1536, (1, 16, 17, 32)), ("q8 q4 t3", 70, 8192, (2, 32)), ("q8 t3", 1600, 6144, (9,)),
+          ("q4 t3", 4128, 1088, (3, 17)), ("q4 t3", 96, 4224, (33, 70)), ("q8 q4 t3", 8230, 64, (3, 32)),
+          ("q8 q4 t3", 17000, 96, (5, 32)), ("q8", 33000, 64, (7,)), ("q4", 100, 768, (40,)), ("q4", 100, 800, (40,)),
+          ("t3", 100, 1024, (16, 17)), ("q8 t3", 9600, 256, (70,)), ("q8 t3", 33000, 64, (40,)), ("q4", 4608, 96, (70,)), ("q4 t3", 9600, 64, (96,)),
+          ("q8 q4 t3", (1 << 22) + 33, 64, (2,))]
+
+
+@pytest.mark.parametrize("kind,rows,cols,ntok", [(k, r, c, n) for ks, r, c, ns in ROUTES for k in ks.split() for n in ns])
+def test_gemm_routes(gpu, kind, rows, cols, ntok):
+    from vgx import mmcf
+    rng = np.random.default_rng(rows + cols + ntok)
+
+    def matrix():  # (any bytes are a matrix; the packers are slow at these sizes)
+        plane = rng.uniform(0.1, 0.9, rows).astype(np.float32)
+        if kind == "q8":
+            return mmcf.Matrix("q8", rows, cols, rng.integers(0, 256, rows * cols, dtype=np.uint8), 1e-3, True, plane)
+        if kind == "t3":
+            body = rng.integers(0, 256, (rows + 1) // 2 * (cols // 8) * 4, dtype=np.uint8)
+            return mmcf.Matrix("t3", rows, cols, body, 2e-2, True, plane)
+        s16, m16 = (rng.integers(-20000, 20000, rows * cols // 32, dtype=np.int16) for _ in range(2))
+        return mmcf.Matrix("q4", rows, cols, rng.integers(0, 256, rows * cols // 2, dtype=np.uint8), 1e-6, s16=s16, m16=m16)
+
+    m1, m3 = matrix(), matrix()
+    W1, W3 = gpu.upload(m1), gpu.upload(m3)
+    x = x_rows(rng, ntok, cols)
+    x[0, :8], x[-1, -8:] = 32767, -32768
+    res = rng.integers(-3000, 3000, (ntok, rows)).astype(np.int16)
+    nw = o.quantize_act(rng.uniform(0.5, 1.5, rows).astype(np.float32)) if rows < 65536 else None
+    half = cols // 64 * 32
+    got, gate = host(gpu.gemm(W1, dev(x), res=dev(res))), host(gpu.ffn_gate_batch(W1, W3, dev(x), 1))
+    got_s = host(gpu.gemm_add_split(W1, half, dev(x), dev(res)))
+    if nw is not None:
+        y, yn = gpu.gemm_norm(W1, dev(x), dev(res), dev(nw), 1e-5)
+        ys, yns = gpu.gemm_norm(W1, dev(x), dev(res), dev(nw), 1e-5, split=half)
+        assert np.array_equal(host(y), got) and np.array_equal(host(ys), got_s)
+    a, b = m1.slice_cols(0, half), m1.slice_cols(half, cols)
+    for t in sorted({0, 1 % ntok, ntok // 2, ntok - 1}):
+        v = oracle_rowval(m1, x[t])
+        assert np.array_equal(got[t], o.store(v, res[t])), t
+        assert np.array_equal(gate[t], o.gate(v, oracle_rowval(m3, x[t]), 1)), t
+        assert np.array_equal(got_s[t], o.store(oracle_rowval(b, x[t, half:]), o.store(oracle_rowval(a, x[t, :half]), res[t]))), t
+        if nw is not None:
+            assert np.array_equal(host(yn)[t], o.rmsnorm(got[t], nw, 1e-5)), t
+            assert np.array_equal(host(yns)[t], o.rmsnorm(got_s[t], nw, 1e-5)), t
+    W1.free()
+    W3.free()
+
+
 @pytest.mark.parametrize("chunk", [32, 8192, 65536])
 def test_gate_every_input(gpu, chunk):
     """The batched gate's table exponential and refined quotient at every one

@@ -27,8 +27,7 @@ struct GemmLaunch {
                             // gridDim.z, an implicit argument whose load would delay the first weights)
 };
 
-// The tile kernel of vgx_gemm.hip over more than one 32-token tile; VGX_ESTATE
-// when no plan of it takes the launch.
+// The tile kernel of vgx_gemm.hip; VGX_ESTATE past its limits on rows and grid.
 int vgx_gemm_tile_launch(const GemmLaunch& L, int epi, int num_cu, hipStream_t s);
 
 namespace {

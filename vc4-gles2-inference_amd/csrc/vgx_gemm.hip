@@ -717,11 +717,6 @@ int vgx_gemm_tile_launch(const GemmLaunch& L, int epi, int num_cu, hipStream_t s
     // the sums' ranges, and 32-bit offsets within a workgroup's rows
     if (L.cols > kMaxCols || L.M.rows > (1 << 22)) return VGX_ESTATE;
     const int kind = L.M.kind;
-    // A q4 launch of one token tile: dequantised into three planes for 32
-    // tokens only, a weight costs more here than its share of the group sums
-    // in the one-tile kernel (32 x 1024 x 4608 two-half residual 14.6 against 11.5 us,
-    // 32 x 768 x 768 6.3 against 5.9); not so the gate, whose epilogue is faster (12.1 -> 10.2).
-    if (kind == VGX_Q4 && L.ntok <= kTile && epi != BEPI_GATE) return VGX_ESTATE;
     const TilePlan P = plan_of(kind, epi, pick_plan(kind, epi, L.M.rows, L.ntok, num_cu));
     const long ntx = (L.M.rows + P.rb - 1) / P.rb, nty = (L.ntok + P.bm - 1) / P.bm;
     const long blocks = (ntx + 7) / 8 * 8 * nty;

@@ -1,6 +1,7 @@
 // Batched GEMM entry points, and the one-token-tile kernel behind the launches
-// that vgx_gemm.hip's tile kernel does not take: the RMSNorm-fused variants,
-// and q4 over at most 32 tokens (the decode of a batch).  Y[t] = W . X[t] for
+// that it runs faster than vgx_gemm.hip's tile kernel (one_tile_faster): the
+// RMSNorm-fused variants, long rows over at most 32 tokens (split over
+// workgroups), and other launches of one token tile.  Y[t] = W . X[t] for
 // ntok token rows with the exact integer sums of the batch-1 GEMV, so every
 // output row is bit-identical to vgx_gemv on that token (the reference's
 // acceptance rule for a batched path: the logits of a grouped prefill equal
@@ -589,32 +590,30 @@ __global__ void __launch_bounds__(kNormThreads) gemm_epi_norm_kernel(const GemmL
 
 using GemmFn = void (*)(const GemmLaunch);
 
-// The RMS variants in every format; without RMS, q4 of one token tile (whole
-// or split) and the shapes past the tile kernel's limits (4 waves).
+// The RMS variants in every format, with 2, 4 or 8 waves.  Without RMS: the split
+// pair in every format; whole rows as one_tile_faster() sends them here, and with
+// two waves the shapes past the tile kernel's limits.
 template <int EPI, int NW, bool RMS, bool PART>
 GemmFn pick_kind(int kind) {
-    switch (kind) {
-        case VGX_Q8: return PART ? nullptr : gemm_kernel<VGX_Q8, EPI, NW, RMS, false>;
-        case VGX_Q4: return gemm_kernel<VGX_Q4, EPI, NW, RMS, PART>;
-        case VGX_T3: return PART ? nullptr : gemm_kernel<VGX_T3, EPI, NW, RMS, false>;
-    }
+    constexpr bool whole = !RMS && !PART;
+    constexpr bool q8 = !whole || NW == 2 || (EPI != BEPI_GATE && NW == 4);
+    constexpr bool t3 = !whole || NW == 2 || EPI != BEPI_SPLIT || NW == 4;
+    constexpr bool q4 = !whole || EPI != BEPI_GATE || NW != 8;
+    if constexpr (q4) if (kind == VGX_Q4) return gemm_kernel<VGX_Q4, EPI, NW, RMS, PART>;
+    if constexpr (q8) if (kind == VGX_Q8) return gemm_kernel<VGX_Q8, EPI, NW, RMS, PART>;
+    if constexpr (t3) if (kind == VGX_T3) return gemm_kernel<VGX_T3, EPI, NW, RMS, PART>;
     return nullptr;
 }
 
 template <int EPI, bool RMS>
 GemmFn pick_nw(int kind, int nw, bool part) {
-    if constexpr (RMS) {
-        switch (nw) {
-            case 2: return pick_kind<EPI, 2, true, false>(kind);
-            case 4: return pick_kind<EPI, 4, true, false>(kind);
-            case 8: return pick_kind<EPI, 8, true, false>(kind);
-        }
-        return nullptr;
-    } else {
-        if (part) return kind == VGX_Q4 ? pick_kind<EPI, 4, false, true>(kind) : nullptr;
-        if (nw == 8) return kind == VGX_Q4 ? gemm_kernel<VGX_Q4, EPI, 8, false, false> : nullptr;
-        return nw == 4 ? pick_kind<EPI, 4, false, false>(kind) : nullptr;
+    if constexpr (!RMS) if (part) return nw == 4 ? pick_kind<EPI, 4, false, true>(kind) : nullptr;
+    switch (nw) {
+        case 2: return pick_kind<EPI, 2, RMS, false>(kind);
+        case 4: return pick_kind<EPI, 4, RMS, false>(kind);
+        case 8: return pick_kind<EPI, 8, RMS, false>(kind);
     }
+    return nullptr;
 }
 
 GemmFn pick(int epi, int kind, int nw, bool rms, bool part) {
@@ -667,21 +666,91 @@ bool workspace(vgx_ctx* ctx, size_t bytes, long long** out) {
     return true;
 }
 
-// Waves per workgroup (measured when every batched launch ran here; now the
-// RMSNorm-fused ones and q4 of one token tile): 4 when the launch has at least one tile per CU (two
+// Waves per workgroup: 4 when the launch has at least one tile per CU (two
 // 4-wave workgroups fit a CU's registers where one 8-wave workgroup does, so
-// up to two tiles a CU run in one round: the 256-token qkv, 384 tiles, took
-// 0.8% less of MiniMind3's 256-token q4 prefill than with 8 waves in two rounds); otherwise (a
-// few row tiles: a decode batch, a short prompt) 8 when the row has more than
-// 16 k-steps, so the tiles' k-steps are spread over more waves.  (16 waves
+// up to two tiles a CU run in one round: 256 tokens of 1,536 x 768 q4, 384 tiles, took
+// 0.8% less of MiniMind3's 256-token q4 prefill than with 8 waves in two rounds);
+// otherwise (a few row tiles: a decode batch, a short prompt) 8 when the row has more
+// than 16 k-steps, so the tiles' k-steps are spread over more waves.  (16 waves
 // would cap a lane at 128 registers and spill the operands in flight; 8 waves
 // with four steps in flight keep as many bytes in flight per CU.)  Above two
 // tiles a CU, 2: four 2-wave workgroups fit a CU, so the launch still runs in
-// one round (the 256-token q4 gate, 608 tiles: 22.5 -> 21.1 us; with 4 waves
-// its last 96 tiles started when the first round ended).
+// one round (608 tiles of a q4 gate of 768 columns: 22.5 -> 21.1 us; with 4 waves
+// its last 96 tiles started when the first round ended).  (The tile kernel now takes
+// the launches of these two figures; an LM head over a batch's rows and the fused
+// norms of more than 32 tokens have as many tiles.)
 int waves_for(int tiles, int nsteps, int num_cu) {
     if (tiles > 2 * num_cu) return 2;
     return tiles < num_cu && nsteps > 16 ? 8 : 4;
+}
+
+// Whether this file's kernel, and with nz > 1 its split pair, takes a launch
+// without RMS from the tile kernel.  It reads a token tile's activations once a
+// workgroup straight into the matrix-core layout and has no barrier in its loop, so it
+// is the better one where the tile kernel's shared operands serve a single token tile,
+// and where the tile kernel's own rounds do not fill.  Both sides in us, this one first.
+//
+// Split (one token tile, few row tiles, rows past 32 k-steps): the tile kernel puts a
+// row tile's K on one CU, the split pair on nz of them and pays a second launch and
+// the partial sums' way through memory.  A k tile of 64 columns on the tile kernel's
+// longest wave is 0.4 us (q8) or 0.6 (t3), the split pair walks c/nz of them, the sums
+// cost 0.7 us a megabyte and the launch 1.7 (store), 2.7 (two halves) or 2.6 (gate).
+// Over 768..2,432 rows x 1..32 tokens x 1,536 to 32,768 columns the side that this
+// takes is the faster one, or slower by up to 10% near the line (0.2% on average).  q8
+// store of 8 tokens x 1,024 rows: 2,048 columns 6.5 / 5.3, 8,192 7.3 / 10.7, 32,768 14 /
+// 34; t3 gate 2 x 768: 1,536 7.3 / 8.0, 4,096 8.0 / 14.5; t3 two halves with the norm,
+// 32 x 1,024 x 4,096: 12.5 / 11.1.  q4 converts each weight into three planes for 32
+// tokens alone and always loses to the pair (gate 8 x 768 x 2,048: 9.2 / 14.5).
+//
+// Whole rows:
+//   store, one token tile of more row tiles than CUs (an LM head): here (8 x 20,000 x
+//     1,024 q8 8.2 / 8.5, 2 x 73,448 20.9 / 26.3; 2 x 64,402 t3 19.0 / 21.6, q4 29 / 42),
+//     but for q8 of 17 tokens and more over four a CU whose 64 x 64 tiles fill
+//     their last round of two a CU (32 x 64,402 25.0 / 22.3; 32 x 73,448 25.9 / 27.7)
+//   q4 of one token tile: here (32 x 768 x 768 5.9 / 6.3), but for the gate of at
+//     most a row tile a CU, whose epilogue is faster there (8 x 4,096 x 1,024 11.0 /
+//     10.2; 2 x 9,600 14.8 / 17.7)
+//   q4 store of few tiles and up to 24 k-steps: here (64 x 1,536 x 768 6.1 / 6.4, 256
+//     columns 4.3 / 5.3; 1,024 columns 6.6 / 6.5)
+//   t3 store up to 16 tokens and 32 k-steps: here (8 x 1,024 x 1,024 4.5 / 4.7; 24
+//     tokens 4.8 / 4.8)
+//   t3 gate up to 16 tokens: here (8 x 4,096 x 1,024 6.4 / 6.9, 4,096 columns 13.3 /
+//     14.5), from 97 k-steps with any number of tokens (64 x 768 x 8,192 22.6 / 24.5),
+//     and one token tile of more row tiles than CUs (2 x 9,600 8.7 / 10.1; q8 only up to
+//     16 tokens past two a CU: 2 x 20,000 x 1,024 13.1 / 14.6, 17 x 9,600 10.2 / 8.3)
+//   q4 and t3 stores whose 64 x 64 tiles would leave a second round nearly empty
+//     (96 x 9,600 x 1,024 q4 15.1 / 20.5, t3 11.0 / 11.6), q4 also where the 64 x 32
+//     ones would (96 x 4,608 x 1,024 10.2 / 11.1)
+//   two halves of up to 16 k-steps in more tiles than CUs: here (256 x 9,600 x 256 q8
+//     17.0 / 22.4, q4 25.6 / 33.3), where the tile kernel's longer epilogue shows
+bool one_tile_faster(int kind, int epi, int ntok, int rows, int nsteps, int nz, int num_cu) {
+    const bool gate = epi == BEPI_GATE, one = ntok <= kTile, q8 = kind == VGX_Q8, q4 = kind == VGX_Q4;
+    if (nz > 1) {
+        if (q4) return true;
+        const int walk = (nsteps + 15) / 16 * (gate ? 2 : 1);
+        const double saved = (q8 ? 0.4 : 0.6) * walk * (1.0 - (gate ? 1.0 : q8 ? 2.0 : 1.5) / nz);
+        const double mbytes = (double)nz * (epi == BEPI_STORE ? 1 : 2) * ntok * rows * 8e-6;
+        return saved > (gate ? 2.6 : epi == BEPI_SPLIT ? 2.7 : 1.7) + 0.7 * mbytes;
+    }
+    // workgroups of the tile kernel's plans
+    const long rt = (rows + kTile - 1) / kTile, t64 = (ntok + 63) / 64;
+    const long b32 = rt * ((ntok + 31) / 32), b64 = rt * t64, b64x64 = (rt + 1) / 2 * t64;
+    const bool few = b32 <= num_cu;
+    if (gate) {
+        if (q4) return one && !few;
+        if (q8) return ntok <= 16 && b32 > 2L * num_cu;
+        return few ? ntok <= 16 || nsteps > 96 : one;
+    }
+    if (q4 && one) return true;
+    if (epi == BEPI_SPLIT) return !few && nsteps <= 16;
+    if (one && !few) {
+        const long rounds = (b64x64 + 2 * num_cu - 1) / (2 * num_cu);
+        return !q8 || ntok <= 16 || b32 <= 4L * num_cu || 4 * b64x64 < (4 * rounds - 1) * 2 * num_cu;
+    }
+    if (q8) return false;
+    if (few) return q4 ? nsteps <= 24 : ntok <= 16 && nsteps <= 32;
+    if (q4 && b32 <= 2L * num_cu) return b64 > num_cu;
+    return b32 <= 4L * num_cu && b64x64 > num_cu;
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -715,24 +784,25 @@ int launch(vgx_ctx* ctx, const vgx_mat* W, const vgx_mat* W3, int ntok, const in
     L.split = split;
     L.rw = rw;
     L.eps = eps;
-    if (!rw) {
-        // (VGX_ESTATE: a launch the tile kernel leaves to this file's)
-        const int st = vgx_gemm_tile_launch(L, epi, ctx->num_cu, ctx->stream);
-        if (st != VGX_ESTATE) return st || !yn ? st : vgx_rmsnorm_batch(ctx, ntok, M.rows, y, nrm_w, neps, yn);
-    }
     dim3 grid((M.rows + kTile - 1) / kTile, (ntok + kTile - 1) / kTile);
     const int nsteps = (M.cols + kTile - 1) / kTile;
     // (the RMS variants stay whole: every split would recompute the row statistics)
-    int nz = rw || M.kind != VGX_Q4 ? 1 : k_splits((int)grid.x, (int)grid.y, nsteps, ctx->num_cu);
-    if (nz > 1) {
+    int nz = rw ? 1 : k_splits((int)grid.x, (int)grid.y, nsteps, ctx->num_cu);
+    if (nz > 1 && one_tile_faster(M.kind, epi, ntok, M.rows, nsteps, nz, ctx->num_cu)) {
         const int na = epi == BEPI_STORE ? 1 : 2;
         const size_t bytes = (size_t)nz * na * ntok * M.rows * sizeof(long long);
         if (!workspace(ctx, bytes, &L.part)) nz = 1;  // no workspace: one pass
-        grid.z = nz;
+    } else {
+        nz = 1;
     }
+    if (!rw && nz == 1 && !one_tile_faster(M.kind, epi, ntok, M.rows, nsteps, 1, ctx->num_cu)) {
+        // (VGX_ESTATE: past the tile kernel's limits)
+        const int st = vgx_gemm_tile_launch(L, epi, ctx->num_cu, ctx->stream);
+        if (st != VGX_ESTATE) return st || !yn ? st : vgx_rmsnorm_batch(ctx, ntok, M.rows, y, nrm_w, neps, yn);
+    }
+    grid.z = nz;
     L.nz = nz;
-    int nw = nz > 1 ? 4 : waves_for((int)(grid.x * grid.y), nsteps, ctx->num_cu);
-    if (!rw && (M.kind != VGX_Q4 || nw == 2)) nw = 4;  // (the variants that exist without RMS)
+    const int nw = nz > 1 ? 4 : waves_for((int)(grid.x * grid.y), nsteps, ctx->num_cu);
     GemmFn fn = pick(epi, M.kind, nw, rw != nullptr, nz > 1);
     if (!fn) return vgx_fail(VGX_EINVAL, std::string(who) + ": unknown weight kind");
     // each wave's activation block (32 tokens x 4 k-steps of 32 int16), then
