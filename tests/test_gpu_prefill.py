@@ -255,6 +255,30 @@ def test_gemm_routes(gpu, kind, rows, cols, ntok):
     W3.free()
 
 
+def test_gemm_past_one_grid_dimension(gpu):
+    """More outputs than workgroups of 512 threads fit along x of a grid (2^32
+    threads): 2,080 tokens of 2^22 rows, 17 GB, written over the residual."""
+    from vgx import mmcf
+    rng = np.random.default_rng(5)
+    rows, cols, ntok, split = 1 << 22, 544, 2080, 256
+    body = rng.integers(0, 256, rows // 2 * (cols // 8) * 4, dtype=np.uint8)
+    m = mmcf.Matrix("t3", rows, cols, body, 2e-2, True, rng.uniform(0.1, 0.9, rows).astype(np.float32))
+    W = gpu.upload(m)
+    x = x_rows(rng, ntok, cols)
+    y = torch.zeros((ntok, rows), dtype=torch.int16, device="cuda")
+    gpu.gemm_add_split(W, split, dev(x), y, out=y)
+    n = 4096  # rows checked at either end
+    zero = np.zeros(n, np.int16)
+    for r0 in (0, rows - n):
+        part = mmcf.Matrix("t3", n, cols, body.reshape(rows // 2, -1)[r0 // 2:(r0 + n) // 2].ravel(), m.scale,
+                           plane=m.plane[r0:r0 + n])
+        a, b = part.slice_cols(0, split), part.slice_cols(split, cols)
+        for t in (0, 1023, ntok - 1):
+            want = o.store(oracle_rowval(b, x[t, split:]), o.store(oracle_rowval(a, x[t, :split]), zero))
+            assert np.array_equal(host(y[t, r0:r0 + n]), want), (r0, t)
+    W.free()
+
+
 @pytest.mark.parametrize("chunk", [32, 8192, 65536])
 def test_gate_every_input(gpu, chunk):
     """The batched gate's table exponential and refined quotient at every one

@@ -720,7 +720,8 @@ int vgx_gemm_tile_launch(const GemmLaunch& L, int epi, int num_cu, hipStream_t s
     const TilePlan P = plan_of(kind, epi, pick_plan(kind, epi, L.M.rows, L.ntok, num_cu));
     const long ntx = (L.M.rows + P.rb - 1) / P.rb, nty = (L.ntok + P.bm - 1) / P.bm;
     const long blocks = (ntx + 7) / 8 * 8 * nty;
-    if (blocks > 0x7FFFFFFFL) return VGX_ESTATE;
+    // (a launch holds less than 2^32 threads along x; the one-tile kernel's grid has a y)
+    if (blocks * P.threads > 0xFFFFFFFFL) return VGX_ESTATE;
     hipLaunchKernelGGL(P.fn, dim3((unsigned)blocks), dim3(P.threads), P.lds, s, L, (int)ntx, (int)nty);
     VGX_LAUNCH_CHECK("gemm tile launch");
     return VGX_OK;

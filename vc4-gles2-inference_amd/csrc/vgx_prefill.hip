@@ -679,7 +679,7 @@ bool workspace(vgx_ctx* ctx, size_t bytes, long long** out) {
 // its last 96 tiles started when the first round ended).  (The tile kernel now takes
 // the launches of these two figures; an LM head over a batch's rows and the fused
 // norms of more than 32 tokens have as many tiles.)
-int waves_for(int tiles, int nsteps, int num_cu) {
+int waves_for(long tiles, int nsteps, int num_cu) {
     if (tiles > 2 * num_cu) return 2;
     return tiles < num_cu && nsteps > 16 ? 8 : 4;
 }
@@ -802,7 +802,7 @@ int launch(vgx_ctx* ctx, const vgx_mat* W, const vgx_mat* W3, int ntok, const in
     }
     grid.z = nz;
     L.nz = nz;
-    const int nw = nz > 1 ? 4 : waves_for((int)(grid.x * grid.y), nsteps, ctx->num_cu);
+    const int nw = nz > 1 ? 4 : waves_for((long)grid.x * grid.y, nsteps, ctx->num_cu);
     GemmFn fn = pick(epi, M.kind, nw, rw != nullptr, nz > 1);
     if (!fn) return vgx_fail(VGX_EINVAL, std::string(who) + ": unknown weight kind");
     // each wave's activation block (32 tokens x 4 k-steps of 32 int16), then
