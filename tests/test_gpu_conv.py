@@ -56,11 +56,12 @@ def test_conv_batch_equals_steps_and_state(gpu):
     C.free()
 
 
-@pytest.mark.parametrize("dim,T", [(64, 2), (1000, 3), (1004, 5), (2056, 4), (1024, 513)])
+@pytest.mark.parametrize("dim,T", [(64, 2), (1000, 3), (1004, 5), (2056, 4), (1024, 513),
+                                   (512, 8), (64, 9), (1000, 9), (1004, 10), (2056, 11)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_conv_batch_shapes(gpu, dim, T, shift):
-    """A batch's parallel kernel at one- and eight-channel widths, odd and even
-    batches, rows that do and do not start on 16 bytes; then the in-place form
+    """Batches either side of the parallel kernel's shortest (9 positions), it at
+    one- and eight-channel widths, odd and even batches, rows that do and do not start on 16 bytes; then the in-place form
     (y over bcx), which walks the positions."""
     import torch
     rng = np.random.default_rng(dim + T)

@@ -82,6 +82,7 @@ __global__ void __launch_bounds__(kThreads) conv_kernel(int dim, int ntok, const
 // the last two gated values themselves), so no workgroup reads what another
 // writes.
 constexpr int kRun = 2;
+constexpr int kWalk = 8;  // positions up to which a batch is walked all the same
 
 template <int V>
 struct __align__(2 * V) Vec {
@@ -218,12 +219,15 @@ int vgx_conv_step(vgx_conv* c, int layer, int ntok, const int16_t* bcx, int16_t*
     const int16_t* taps = c->taps + (size_t)layer * 3 * c->dim;
     int16_t* st = c->state + (size_t)layer * 2 * c->dim;
     // A batch runs its positions in parallel, 8 channels a thread where every
-    // row starts on 16 bytes.  One position, and rows written over bcx (each
-    // channel's walk reads a value before it is overwritten), keep the walk.
+    // row starts on 16 bytes.  Rows written over bcx (each channel's walk reads a
+    // value before it is overwritten) keep the walk, and so do a few positions,
+    // whose walk is over within the cost of a launch.  us, walk against parallel: 4
+    // positions of 64 channels 3.0 / 3.4, of 1,024 3.0 / 3.3, of 8,192 3.0 / 3.7; 8 of
+    // 1,024 3.2 / 3.3; 10 of 1,024 3.6 / 3.3; 17 of 1,024 5.2 / 3.5.
     const size_t yn = (size_t)ntok * c->dim;
     const bool apart = y + yn <= bcx || bcx + 3 * yn <= y;
     const unsigned runs = ((unsigned)ntok + kRun - 1) / kRun;
-    if (ntok > 1 && apart && runs <= 65535u) {
+    if (ntok > kWalk && apart && runs <= 65535u) {
         const bool wide = c->dim % 8 == 0 && (((uintptr_t)bcx | (uintptr_t)y) & 15u) == 0;
         const int per = wide ? c->dim / 8 : c->dim;
         // whole waves, no more than the channels need
