@@ -363,6 +363,22 @@ def test_batches_around_one_round(gpu, bits, heads, kvh, hd, seq, batches, rails
     test_tile_attention_batches(gpu, bits, heads, kvh, hd, seq, batches, rails)
 
 
+# The same for a q8 cache's two workgroups a CU around 512 positions, one and a half
+# rounds beside tile workgroups of 16 heads, and four query vectors of wide heads.
+LINES = [(8, 16, 16, 32, 600, ((480, 32), (481, 32), (560, 17)), False),
+         (8, 8, 8, 160, 600, ((464, 48), (465, 48)), True),
+         (8, 8, 4, 96, 600, ((540, 48),), False),
+         (16, 16, 1, 64, 320, ((250, 33), (200, 48), (200, 49)), False),
+         (16, 32, 1, 32, 320, ((232, 24), (233, 24), (270, 25)), True),
+         (16, 32, 8, 128, 160, ((0, 17), (100, 33)), False),
+         (16, 32, 8, 112, 160, ((0, 24), (100, 40)), True)]
+
+
+@pytest.mark.parametrize("bits,heads,kvh,hd,seq,batches,rails", LINES)
+def test_batches_around_the_lines(gpu, bits, heads, kvh, hd, seq, batches, rails):
+    test_tile_attention_batches(gpu, bits, heads, kvh, hd, seq, batches, rails)
+
+
 @pytest.mark.parametrize("bits,heads,kvh,hd,counts", [(16, 16, 2, 64, (16, 17, 32, 33)), (8, 16, 8, 64, (16, 17, 32)),
                                                       (16, 8, 4, 96, (32, 34, 64, 65)), (8, 32, 1, 128, (8, 9, 17))])
 def test_sequences_around_one_round(gpu, bits, heads, kvh, hd, counts):

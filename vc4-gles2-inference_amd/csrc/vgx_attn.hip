@@ -1976,7 +1976,17 @@ size_t group_plan(const AttnDev& A, bool seqs, int pos0, int n, int num_cu, Grou
 // rows of 16 heads of 64 at 460 (two workgroups on some CUs) 10.9 / 13.3; 32 of
 // them at 500 12.7 / 15.8, at 4,000 50.8 / 64.8.  With one more round it is no
 // longer so (33 rows at 0 9.8 / 9.0; a q8 cache with heads of 64, whose instance
-// has one workgroup a CU, 17 rows at 300 13.1 / 10.5).
+// has one workgroup a CU, 17 rows at 300 13.1 / 10.5), with two exceptions:
+//   A q8 cache with two workgroups on a CU gains less, and past about 512 positions
+//   nothing where few query vectors would share a workgroup (groups of up to 4 heads),
+//   but for heads of 65 to 96, whose instance holds a K row in three slots: 32 rows of
+//   16 heads of 16 at 480 10.8 / 11.5, at 3,900 52.4 / 47.2; 48 of 8 of 256 at 250 16.8 /
+//   17.6, at 3,900 143 / 137; 48 of 8 of 96 at 3,900 60 / 75.
+//   At a q16 cache with 16 heads a tile workgroup, those are few and long, and past
+//   256 positions up to one and a half rounds of the per-head kernel are over before
+//   them: 33 rows of 16 heads of 64 over one KV head at 250 12.8 / 14.8, 48 at 1,000
+//   26.1 / 30.7; 24 of 32 heads of 32 at 200 11.4 / 10.4, at 1,000 21.3 / 24.7; 48 of 16
+//   of 128 at 480 23.7 / 28.8.
 //
 // Sequences each have a cache of their own, so two workgroups on a CU share its
 // bandwidth: they keep to it as long as what the launch reads comes to at most
@@ -1986,9 +1996,13 @@ size_t group_plan(const AttnDev& A, bool seqs, int pos0, int n, int num_cu, Grou
 bool heads_at_once(const vgx_attn* at, bool seqs, int pos, int n) {
     const AttnDev& A = at->a;
     const int num_cu = at->ctx->num_cu;
-    const long blocks = (long)A.heads * n;
-    if (blocks > (long)num_cu * at->per_cu) return false;
-    if (!seqs || blocks <= num_cu || blocks * (pos + 1) * 2 * A.pstride <= (long)num_cu * (128 << 10)) return true;
+    const long blocks = (long)A.heads * n, slots = (long)num_cu * at->per_cu;
+    // (tile workgroups of 16 heads: launch_tile halves a group of 16, 32, .. to 16)
+    const bool tile16 = !seqs && A.kv_bits == 16 && A.hd <= 128 && A.group % 16 == 0 && (A.group & (A.group - 1)) == 0;
+    if (blocks > slots) return tile16 && 2 * blocks <= 3 * slots && pos + n > 256;
+    if (blocks <= num_cu) return true;
+    if (!seqs) return A.kv_bits == 16 || A.group > 4 || (A.hd > 64 && A.hd <= 96) || pos + n <= 512;
+    if (blocks * (pos + 1) * 2 * A.pstride <= (long)num_cu * (128 << 10)) return true;
     GroupArgs g{};
     return !group_plan(A, true, pos, n, num_cu, g) || (long)A.kv_heads * (A.group / g.hs) * n > num_cu;
 }
@@ -2059,8 +2073,9 @@ int launch_tile(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv, 
     // phases win.  It runs one V pass up to 4, two up to 8; us at position 500, it
     // against this kernel: heads of 64, q8 cache, 2 vectors 13.1 / 17.1, 4 16.8 / 17.4,
     // 6 22.2 / 17.7; q16 4 20.2 / 18.1, 6 26.7 / 18.4; heads of 96, q8 4 21.2 / 21.5, 6
-    // 33.8 / 24.3; q16 4 25.3 / 22.8, 6 38.6 / 25.8.
-    if (g.hs * g.tq < (A.kv_bits == 16 ? 4 : 5)) return VGX_ESTATE;
+    // 33.8 / 24.3; q16 4 25.3 / 22.8, 6 38.6 / 25.8; q16 at 250, 4 vectors: heads of 112
+    // 16.9 / 19.8, of 128 18.8 / 20.5.
+    if (g.hs * g.tq < (A.kv_bits == 16 && A.hd <= 96 ? 4 : 5)) return VGX_ESTATE;
     g.nby = (ntok + g.tq - 1) / g.tq;
     if (g.nby > 65535) return VGX_ESTATE;
     g.nw = std::max(8, A.hd / 8);
