@@ -406,8 +406,8 @@ def test_sequences_around_one_round(gpu, bits, heads, kvh, hd, counts):
 def test_exp_tables_round_as_exp():
     """The tile kernel's exp(-k/1024) = T[k >> 8] * U[k & 255] and the batched
     gate's exp(-g/256) = T'[(g >> 8) + 128] * U'[g & 255], as floats: over every
-    argument the exact value keeps 2^-44 away from a float rounding boundary,
-    four hundred times what two factors and a product in double can err."""
+    argument the exact value keeps 2^-44 of itself away from a float rounding
+    boundary, about a hundred times what two factors and a product in double can err."""
     for x in (-np.arange(65536, dtype=np.longdouble) / 1024, -np.arange(-32768, 32768, dtype=np.longdouble) / 256):
         e = np.exp(x)
         with np.errstate(over="ignore"):
@@ -419,3 +419,36 @@ def test_exp_tables_round_as_exp():
             assert (np.abs(e - mid)[ok] / e[ok]).min() > 2.0 ** -44
         # past the float range on either side by more than that
         assert not np.any(f[~ok & (x < 0)]) and np.all(np.isinf(f[~ok & (x > 0)]) | (x[~ok & (x > 0)] > 88))
+
+
+def test_tile_exponential_every_distance(gpu):
+    """The tile kernel over every score distance k = 0..65535: a query of 8.0 in
+    one element and K rows whose element is 32767 (position 0) and 32767 - k (the
+    rows, each head its own 512 distances), no rotation.  Every row equals the
+    per-head kernel, which takes exp in double, and the first, a middle and the last
+    the oracle."""
+    heads, hd, n = 64, 16, 513
+    dim = heads * hd
+    rc, rs = np.ones((n, hd // 2), np.float32), np.zeros((n, hd // 2), np.float32)
+    A = gpu.attention(dim=dim, heads=heads, kv_heads=heads, head_dim=hd, seq=n, layers=1, kv_bits=16, rope_half=1,
+                      qk_norm=0, rope_cos=rc, rope_sin=rs)
+    c, rtab = o.attn_cfg(dim, heads, heads, hd, n, 16, 1, 0), o.rope_table(rc, rs)
+    rng = np.random.default_rng(3)
+    for base in (0, 32768):
+        x = np.zeros((n, 3, heads, hd), np.int16)
+        x[:, 0, :, 0] = 2048
+        x[0, 1, :, 0] = 32767
+        k = base + np.arange(512)[:, None] + 512 * np.arange(heads)[None, :]
+        x[1:, 1, :, 0] = 32767 - k
+        x[1:, 2] = rng.integers(0, 32768, (512, heads, hd))
+        x = x.reshape(n, 3 * dim)
+        X = dev(x)
+        got = A.block_batch(0, 0, X)
+        for t in range(n):
+            assert torch.equal(A.decode(0, t, X[t]), got[t]), (base, t)
+        got = got.cpu().numpy()
+        assert base or len(np.unique(got)) > 1000  # (the weights are seen)
+        for t in (0, 256, 512):
+            kv = A.read_rows(0, 0, n).copy()
+            assert np.array_equal(got[t], o.attn_block(c, x[t], None, None, rtab, t, kv)), (base, t)
+    A.free()

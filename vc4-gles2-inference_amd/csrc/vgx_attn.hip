@@ -1397,8 +1397,8 @@ __global__ void __launch_bounds__(kThreads) attn_group_kernel(const AttnDev A, c
 //   scores   q . k by v_mfma_i32_16x16x64_i8 over byte planes, a wave per 16
 //            positions: the exact integer of the dot products
 //   exp      exp(-k/1024) of an integer k in 0..65535 as the product of two
-//            256-entry tables of doubles: no exp(-k/1024) lies within 2^-39 of a
-//            float rounding boundary (over all 65536), and the product is
+//            256-entry tables of doubles: no exp(-k/1024) lies within 2^-40 of
+//            itself of a float rounding boundary (over all 65536), and the product is
 //            within 2^-50, so the float is the one of exp in double
 //   V        v_mfma_f64_16x16x4_f64, a wave per 16 elements: it accumulates its
 //            four positions by fused multiply-adds in position order (checked bit
@@ -1429,13 +1429,6 @@ struct TileArgs {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef double v4d __attribute__((ext_vector_type(4)));
-
-// Global loads stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 template <int KVB, int KS>
 __global__ void __launch_bounds__(512 * KS, 4) attn_tile_kernel(const AttnDev A, const TileArgs g) {
@@ -1989,10 +1982,17 @@ size_t group_plan(const AttnDev& A, bool seqs, int pos0, int n, int num_cu, Grou
 //   of 128 at 480 23.7 / 28.8.
 //
 // Sequences each have a cache of their own, so two workgroups on a CU share its
-// bandwidth: they keep to it as long as what the launch reads comes to at most
-// 128 KB a CU (32 sequences of 16 heads of 64: at 130 8.3 / 10.0, at 255 9.3 /
-// 10.5, at 270 11.5 / 11.8, at 320 13.7 / 12.1), or the query-block kernel, one
-// workgroup a CU, would need a second round (17 sequences at 255 8.9 / 18.0).
+// bandwidth: they keep to it as long as what the workgroups read comes to at most
+// 128 KB a CU, each query head's reads counted, or the query-block kernel, one
+// workgroup a CU, would need a second round (17 sequences of 16 heads of 64 over 2 at
+// 255 8.9 / 18.0).  The line, per-head / query-block by KB a CU, where that kernel
+// fills one round:
+//   16 heads of 64 over 2 or 8, q16, 32 sequences: 112 8.8 / 10.3, 128 9.3 / 10.4,
+//     135 11.5 / 11.8, 144 12.6 / 11.8
+//   8 of 96 over 4, 64: q16 120 9.7 / 11.0, 144 11.3 / 11.1; q8 120 11.8 / 12.6, 132
+//     12.8 / 12.8, 144 13.6 / 12.9
+//   32 of 128 over 8, q16, 16: 128 9.0 / 10.1, 160 13.0 / 11.4
+//   32 of 32 over 4, q16, 16: 128 10.8 / 12.5, 160 15.8 / 14.4
 bool heads_at_once(const vgx_attn* at, bool seqs, int pos, int n) {
     const AttnDev& A = at->a;
     const int num_cu = at->ctx->num_cu;
@@ -2055,9 +2055,9 @@ TileKernel tile_kernel(int kvb, int ks) {
 }
 
 // The tile kernel over rows 0..ntok-1 (positions pos .. pos+ntok-1), as many
-// rows a workgroup as leave about one a CU; VGX_ESTATE when its score rows do
-// not fit the LDS (about 1,500 positions and up), past head_dim 128, and for
-// blocks of few query vectors.
+// rows a workgroup as leave about one a CU; VGX_ESTATE when its 16 score rows do
+// not fit the LDS (past 2,080 positions at head_dim 16, 1,728 at 64, 1,472 at 96,
+// 1,216 at 128), past head_dim 128, and for blocks of few query vectors.
 int launch_tile(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv, int16_t* out) {
     const AttnDev& A = at->a;
     if (A.hd > 128) return VGX_ESTATE;

@@ -38,14 +38,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void keep(u32x4& x) { asm volatile("" : "+v"(x)); }
 
-// The LDS barrier of a tile: this wave's LDS accesses are done, then every
-// wave's.  Global loads stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // 16-byte piece q of LDS row r (of BYTES) lies at q ^ swz_row(r): the 16 rows
 // that one step of a wave's read covers spread over all banks.
 template <int BYTES>
@@ -169,9 +161,9 @@ __device__ __forceinline__ int q16_med(float v) {
 
 // gate_value * 2^0 with exp(-g/256) from two 256-entry tables of doubles,
 // e[0..255] = exp(128 - i) and e[256..511] = exp(-i/256), and f = 2^(8 - hs).
-// The factors and their product are each within 2^-52, and over all 65536 g
-// no exp(-g/256) lies within 2^-43 of a float rounding boundary, so the float
-// is the one of exp in double.  The quotient: a reciprocal refined once, then
+// The factors and their product are each within 2^-52, and over all 65536 g no
+// exp(-g/256) lies within 2^-44 of itself of a float rounding boundary, so the
+// float is the one of exp in double.  The quotient: a reciprocal refined once, then
 // the quotient corrected by its exact remainder (Markstein), which is the
 // correctly rounded one for every g; past 2^100 the factor is cut off, where the
 // product rounds to 0 all the same.

@@ -1,5 +1,5 @@
 // Device helpers shared by the GEMV, GEMM, norm and attention kernels: the
-// byte dot products, the q16 store rounding, the RMSNorm output element and
+// LDS barrier, the byte dot products, the q16 store rounding, the RMSNorm output element and
 // the byte planes of a q16 activation chunk.  Every kernel that reproduces a
 // GEMV row or a normalised activation uses these same expressions, so the
 // paths stay bit-identical.
@@ -10,6 +10,14 @@
 #pragma clang fp contract(off)
 
 namespace {
+
+// The LDS barrier of a workgroup: this wave's LDS accesses are done, then every
+// wave's.  Global loads stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
     return __builtin_amdgcn_sdot4((int)a, (int)b, c, false);
