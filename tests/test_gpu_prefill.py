@@ -41,10 +41,8 @@ def test_gemm_rows_equal_gemv(gpu, kind, rows, cols, ntok):
 @pytest.mark.parametrize("kind,rows,cols", [("q8", 1536, 768), ("q4", 1536, 768), ("t3", 1280, 1024),
                                             ("q4", 768, 2432), ("q8", 2432, 768)])
 def test_gemm_256_tokens(gpu, kind, rows, cols):
-    """The prefill launches of 256 tokens: four waves a workgroup over many
-    tiles (eight over the 2432-column rows' few), each wave's k-steps in
-    rounds of eight, the last token tile ragged at 250 tokens; every row
-    equals the batch-1 oracle."""
+    """The prefill launches of 256 tokens, the last token tile ragged at 250
+    tokens; every row equals the batch-1 oracle."""
     rng = np.random.default_rng(rows * 3 + cols)
     m = MK[kind](rng, rows, cols)
     W = gpu.upload(m)
@@ -102,12 +100,13 @@ def test_ffn_gate_batch(gpu, kind, rows, cols):
             assert np.array_equal(got[t], want), (hs, t)
 
 
-# The tile kernel's plans by output tiles of 32 x 32 (rows/32 x tokens/32: up to
-# one a CU, 2.2, 3.5, 6 and more at 256 CUs), with ragged rows and tokens, a row of
-# one k-step and rows that end inside a k tile, past one K group's run or before
-# the last group's; the split column off a k-step where the format allows it.
+# The tile kernel's plans by the workgroups each would have (32 x 32, 64 x 32 and 128 x
+# 32 outputs, at 256 CUs): up to one a CU of each, two, and more, with ragged rows and
+# tokens, a row of one k-step and rows that end inside a k tile, past one K group's run
+# or before the last group's; the split column off a k-step where the format allows it.
 @pytest.mark.parametrize("kind", ["q8", "q4", "t3"])
-@pytest.mark.parametrize("rows,ntok", [(33, 33), (2100, 70), (4130, 97), (6150, 97), (9650, 97), (13000, 129)])
+@pytest.mark.parametrize("rows,ntok", [(33, 33), (2100, 70), (2432, 117), (4608, 96), (4130, 97), (6150, 97), (9650, 97),
+                                       (13000, 129)])
 @pytest.mark.parametrize("cols_unit", [1, 3, 19])
 def test_gemm_tile_plans(gpu, kind, rows, ntok, cols_unit):
     rng = np.random.default_rng(rows + ntok + cols_unit)
@@ -431,9 +430,9 @@ def test_gemm_q4_adversarial_groups(gpu):
 
 
 # Launches of one token tile whose row tiles leave most CUs idle (the decode
-# batch) split K across workgroups: each stores its exact integer sums and an
-# epilogue kernel adds them and applies the fp32 epilogue -- every row still
-# equals the oracle's batch-1 result
+# batch) may split K across workgroups (q4 past 1,024 columns, q8 and t3 where it
+# pays): each stores its exact integer sums and an epilogue kernel adds them and
+# applies the fp32 epilogue -- every row still equals the oracle's batch-1 result
 @pytest.mark.parametrize("kind,rows,cols", [("q8", 768, 2432), ("q4", 768, 2432), ("t3", 1024, 4096),
                                             ("t3", 1280, 1024), ("q4", 1536, 768)])
 @pytest.mark.parametrize("ntok", [1, 7, 32])
@@ -463,13 +462,15 @@ def test_split_k_decode_batch(gpu, kind, rows, cols, ntok):
 
 
 @pytest.mark.parametrize("kind,rows,cols", [("t3", 1024, 1024), ("q8", 768, 2432), ("q4", 768, 768),
-                                            ("t3", 1024, 4096), ("q8", 1040, 2432)])
+                                            ("t3", 1024, 4096), ("q8", 1040, 2432), ("q4", 768, 2432),
+                                            ("q4", 1024, 4096), ("q4", 1040, 2432), ("q8", 1040, 8192),
+                                            ("t3", 768, 8192)])
 @pytest.mark.parametrize("ntok", [1, 32, 40])
 def test_gemm_norm_equals_gemm_then_rmsnorm(gpu, kind, rows, cols, ntok):
     # the GEMM that writes the residual stream and the RMSNorm of its rows:
-    # in the split-K epilogue launch (32 rows or fewer and rows longer than 32
-    # k-steps: norm slices of 24, 32 and 33 values) or as a launch of its own
-    # (40 rows, or K = 1024), the same bytes as vgx_gemm / vgx_gemm_add_split
+    # in the split-K epilogue launch (32 tokens or fewer of q4 past 32 k-steps and
+    # of the longer q8 and t3 rows: norm slices of 24, 32 and 33 values) or as a
+    # launch of its own (the others), the same bytes as vgx_gemm / vgx_gemm_add_split
     # then vgx_rmsnorm_batch, and the oracle's rows
     rng = np.random.default_rng(rows + ntok)
     m = MK[kind](rng, rows, cols)
