@@ -38,12 +38,11 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void keep(u32x4& x) { asm volatile("" : "+v"(x)); }
 
-// 16-byte piece q of LDS row r (of BYTES) lies at q ^ swz_row(r): the 16 rows
-// that one step of a wave's read covers spread over all banks.
-template <int BYTES>
-__device__ __forceinline__ int swz_row(int r) {
-    return BYTES == 128 ? (r >> 1) & 7 : (r >> 2) & 3;
-}
+constexpr int KS = 2;  // k-steps (32 columns) of a k tile
+
+// 16-byte piece q of LDS row r (of 32 * KS bytes) lies at q ^ swz_row(r): the 16
+// rows that one step of a wave's read covers spread over all banks.
+__device__ __forceinline__ int swz_row(int r) { return (r >> 2) & 3; }
 
 __device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t r, int off) {
     return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
@@ -224,7 +223,7 @@ __device__ __forceinline__ void sums_to_float(const Sum<KIND> (&S)[N], float (&f
     }
 }
 
-template <int KIND, int EPI, int MT, int NT, int WM, int WN, int WK, int KS>
+template <int KIND, int EPI, int MT, int NT, int WM, int WN, int WK>
 struct Tile {
     static constexpr int threads = 64 * WM * WN * WK, gt = 64 * WM * WN;  // of the block, of a K group
     static constexpr int bm = kTile * MT * WM, bk = kTile * KS, wrows = kTile * NT * WN;
@@ -234,8 +233,8 @@ struct Tile {
     static constexpr bool solo = WM * WN == 1;                // a wave stages its own operands
     static constexpr int buf = bm * bk * 2 + wrows * bk * planes;
     static constexpr int stage = buf * WK * (solo ? 1 : 2);
-    // each output's sums lie in one wave: no exchange through LDS
-    static constexpr bool direct = WK == 1 && (EPI == BEPI_STORE || (EPI == BEPI_GATE && NT == 2));
+    // each output's sums (W1's and W3's) lie in one wave: no exchange through LDS
+    static constexpr bool direct = WK == 1 && EPI == BEPI_GATE && NT == 2;
     static constexpr int red = direct ? 0 : WM * WN * WK * NT * 16 * 64 * 8;
     static constexpr int lds = (stage > red ? stage : red) + WK * wrows * 8 + (EPI == BEPI_GATE ? 4096 : 0);
     static constexpr bool ok = bm * 2 * KS % gt == 0 && wrows * 2 * KS % gt == 0 && rt * kTile * kTile * WM % threads == 0 &&
@@ -245,11 +244,10 @@ struct Tile {
 
 // MT x NT: 32-token and 32-row tiles a wave (the gate: NT = 2 holds W1 and W3
 // of the same rows, NT = 1 alternates them over the waves).  WM x WN waves a K
-// group, WK groups (the split: half of them on each column half).  KS: k-steps
-// (32 columns) of a k tile.
-template <int KIND, int EPI, int MT, int NT, int WM, int WN, int WK, int KS>
+// group, WK groups (the split: half of them on each column half).
+template <int KIND, int EPI, int MT, int NT, int WM, int WN, int WK>
 __global__ void __launch_bounds__(64 * WM * WN * WK, WM* WN* WK <= 4 ? 2 : 1) gemm_tile_kernel(const GemmLaunch G, int ntx, int nty) {
-    using T = Tile<KIND, EPI, MT, NT, WM, WN, WK, KS>;
+    using T = Tile<KIND, EPI, MT, NT, WM, WN, WK>;
     constexpr int NC = KIND == VGX_Q4 ? 4 : 2;  // int32 accumulators of an output
     constexpr int BK = T::bk, BM = T::bm, RT = T::rt, NTH = T::threads;
     extern __shared__ __align__(16) unsigned char s_dyn[];
@@ -353,7 +351,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK, WM* WN* WK <= 4 ? 2 : 1) ge
                                    xr[p][1].x, xr[p][1].y, xr[p][1].z, xr[p][1].w};
             uint32_t h[4], l[4];
             planes16(d, h, l);
-            unsigned char* at = xb + row * BK + ((q ^ swz_row<BK>(row)) << 4);
+            unsigned char* at = xb + row * BK + ((q ^ swz_row(row)) << 4);
             *reinterpret_cast<uint4*>(at) = make_uint4(h[0], h[1], h[2], h[3]);
             *reinterpret_cast<uint4*>(at + BM * BK) =
                 make_uint4(l[0] ^ 0x80808080u, l[1] ^ 0x80808080u, l[2] ^ 0x80808080u, l[3] ^ 0x80808080u);
@@ -365,14 +363,14 @@ __global__ void __launch_bounds__(64 * WM * WN * WK, WM* WN* WK <= 4 ? 2 : 1) ge
             int ws;
             w_ops<KIND>(wr[k], row, w, ws);
             wsum[k] += count ? ws : 0;
-            unsigned char* at = wb + row * BK + ((q ^ swz_row<BK>(row)) << 4);
+            unsigned char* at = wb + row * BK + ((q ^ swz_row(row)) << 4);
 #pragma unroll
             for (int c = 0; c < T::planes; ++c)
                 *reinterpret_cast<uint4*>(at + c * T::wrows * BK) = make_uint4(w[c].d[0], w[c].d[1], w[c].d[2], w[c].d[3]);
         }
     };
     auto frag = [&](const unsigned char* plane, int row, int s, Op& o) {
-        const uint4 v = *reinterpret_cast<const uint4*>(plane + row * BK + (((2 * s + half) ^ swz_row<BK>(row)) << 4));
+        const uint4 v = *reinterpret_cast<const uint4*>(plane + row * BK + (((2 * s + half) ^ swz_row(row)) << 4));
         o.d[0] = v.x; o.d[1] = v.y; o.d[2] = v.z; o.d[3] = v.w;
     };
     // the tile's products; next: the next tile is staged between them (the
@@ -479,54 +477,29 @@ __global__ void __launch_bounds__(64 * WM * WN * WK, WM* WN* WK <= 4 ? 2 : 1) ge
     const float gf = EPI == BEPI_GATE ? ldexpf(256.0f, -G.hs) : 0.0f;
 
     if constexpr (T::direct) {
-        // every output's sums are in this wave's registers
-        constexpr int NJ = EPI == BEPI_GATE ? 1 : NT;
-        float sc[NT];
-        int col[NJ];  // byte offset of the output column (a row past the matrix: past the buffer)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            const int o = n0 + (EPI == BEPI_GATE ? wn : wn * NT + j) * kTile + li;
-            if (j < NJ) col[j] = o < rows ? o * 2 : kPast;
-            const MatDev& M = EPI == BEPI_GATE && j == 1 ? G.M3 : G.M;
-            sc[j] = KIND == VGX_Q4 ? M.ps : M.wsr[min(o, rows - 1)];
-        }
-        // output r of token tile m: byte offset of its token's row
-        auto row_of = [&](int m, int r) { return ((wm * MT + m) * kTile + 8 * (r >> 2) + 4 * half + (r & 3)) * G.ldy * 2; };
-        auto at = [&](int j, int ro) { return col[j] == kPast ? kPast : ro + col[j]; };
-        int rs[2][NJ][16];
-        auto res_load = [&](int m) {
-            if (EPI == BEPI_GATE) return;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    rs[m & 1][j][r] = (int)(int16_t)__builtin_amdgcn_raw_buffer_load_b16(rrs, at(j, row_of(m, r)), 0, 0);
-        };
-        res_load(0);
+        // W1's sums and W3's of the same outputs are in this wave's registers
+        const int o = n0 + wn * kTile + li, oc = min(o, rows - 1);
+        const float sc = KIND == VGX_Q4 ? G.M.ps : G.M.wsr[oc], sc3 = KIND == VGX_Q4 ? G.M3.ps : G.M3.wsr[oc];
         __syncthreads();
-        WSum wt[NT];
-#pragma unroll
-        for (int j = 0; j < NT; ++j) wt[j] = s_ws[(wn * NT + j) * kTile + li];
+        const WSum wt = s_ws[wn * NT * kTile + li], wt3 = s_ws[(wn * NT + 1) * kTile + li];
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            if (m + 1 < MT) res_load(m + 1);
-            float v[NT][16];
+            float v[16], v3[16];
+            Sum<KIND> S[16], S3[16];
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                Sum<KIND> S[16];
-#pragma unroll
-                for (int r = 0; r < 16; ++r) S[r] = sum_of(m, j, r, wt[j]);
-                sums_to_float<KIND, 16>(S, v[j]);
+            for (int r = 0; r < 16; ++r) {
+                S[r] = sum_of(m, 0, r, wt);
+                S3[r] = sum_of(m, 1, r, wt3);
             }
+            sums_to_float<KIND, 16>(S, v);
+            sums_to_float<KIND, 16>(S3, v3);
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float a = v[j][r] * sc[j];
-                    const int o = EPI == BEPI_GATE ? q16_med(gate_value_tab(a, v[NT - 1][r] * sc[NT - 1], gf, s_e))
-                                                   : q16_med(a + (float)rs[m & 1][j][r]);  // (no residual: a + 0.0f = a)
-                    __builtin_amdgcn_raw_buffer_store_b16((short)o, yrs, at(j, row_of(m, r)), 0, 0);
-                }
+            for (int r = 0; r < 16; ++r) {
+                // token 8*(r/4) + 4*half + r%4 of the tile (a row past the matrix: past the buffer)
+                const int t = (wm * MT + m) * kTile + 8 * (r >> 2) + 4 * half + (r & 3);
+                __builtin_amdgcn_raw_buffer_store_b16((short)q16_med(gate_value_tab(v[r] * sc, v3[r] * sc3, gf, s_e)), yrs,
+                                                      o < rows ? (t * G.ldy + o) * 2 : kPast, 0, 0);
+            }
         }
         return;
     }
@@ -603,11 +576,11 @@ struct TilePlan {
     int bm, rb, threads, lds;
 };
 
-template <int KIND, int EPI, int MT, int NT, int WM, int WN, int WK, int KS>
+template <int KIND, int EPI, int MT, int NT, int WM, int WN, int WK>
 TilePlan plan() {
-    using T = Tile<KIND, EPI, MT, NT, WM, WN, WK, KS>;
+    using T = Tile<KIND, EPI, MT, NT, WM, WN, WK>;
     if constexpr (T::ok && !(KIND == VGX_Q4 && MT * NT > 2))
-        return TilePlan{gemm_tile_kernel<KIND, EPI, MT, NT, WM, WN, WK, KS>, T::bm, kTile * T::rt, T::threads, T::lds};
+        return TilePlan{gemm_tile_kernel<KIND, EPI, MT, NT, WM, WN, WK>, T::bm, kTile * T::rt, T::threads, T::lds};
     else return TilePlan{};
 }
 
@@ -633,20 +606,20 @@ template <int KIND>
 TilePlan plan_of(int epi, int i) {
     constexpr bool q4 = KIND == VGX_Q4;
     if (epi == BEPI_STORE) switch (i) {
-        case 0: return plan<KIND, BEPI_STORE, 1, 1, 1, 1, 8, 2>();
-        case 1: return plan<KIND, BEPI_STORE, 1, 1, 2, 1, 4, 2>();
-        case 2: return plan<KIND, BEPI_STORE, 1, 1, 2, 2, 2, 2>();
+        case 0: return plan<KIND, BEPI_STORE, 1, 1, 1, 1, 8>();
+        case 1: return plan<KIND, BEPI_STORE, 1, 1, 2, 1, 4>();
+        case 2: return plan<KIND, BEPI_STORE, 1, 1, 2, 2, 2>();
     }
     if (epi == BEPI_SPLIT) switch (i) {
-        case 0: return plan<KIND, BEPI_SPLIT, 1, 1, 1, 1, 8, 2>();
-        case 1: return plan<KIND, BEPI_SPLIT, 2, 1, 1, 1, 8, 2>();
+        case 0: return plan<KIND, BEPI_SPLIT, 1, 1, 1, 1, 8>();
+        case 1: return plan<KIND, BEPI_SPLIT, 2, 1, 1, 1, 8>();
     }
     if (epi == BEPI_GATE) switch (i) {
-        case 0: return plan<KIND, BEPI_GATE, 1, 1, 1, 2, 4, 2>();
-        case 1: return plan<KIND, BEPI_GATE, 1, 1, 2, 2, 2, 2>();
-        case 2: if constexpr (q4) return plan<KIND, BEPI_GATE, 2, 1, 2, 2, 2, 2>(); else break;
-        case 3: return plan<KIND, BEPI_GATE, 1, 1, 2, 2, 1, 2>();
-        case 4: if constexpr (!q4) return plan<KIND, BEPI_GATE, 1, 2, 2, 2, 1, 2>(); else break;
+        case 0: return plan<KIND, BEPI_GATE, 1, 1, 1, 2, 4>();
+        case 1: return plan<KIND, BEPI_GATE, 1, 1, 2, 2, 2>();
+        case 2: if constexpr (q4) return plan<KIND, BEPI_GATE, 2, 1, 2, 2, 2>(); else break;
+        case 3: return plan<KIND, BEPI_GATE, 1, 1, 2, 2, 1>();
+        case 4: if constexpr (!q4) return plan<KIND, BEPI_GATE, 1, 2, 2, 2, 1>(); else break;
     }
     return TilePlan{};
 }
