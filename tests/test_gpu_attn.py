@@ -371,7 +371,9 @@ LINES = [(8, 16, 16, 32, 600, ((480, 32), (481, 32), (560, 17)), False),
          (16, 16, 1, 64, 320, ((250, 33), (200, 48), (200, 49)), False),
          (16, 32, 1, 32, 320, ((232, 24), (233, 24), (270, 25)), True),
          (16, 32, 8, 128, 160, ((0, 17), (100, 33)), False),
-         (16, 32, 8, 112, 160, ((0, 24), (100, 40)), True)]
+         (16, 32, 8, 112, 160, ((0, 24), (100, 40)), True),
+         (8, 20, 4, 64, 160, ((0, 28), (100, 51)), False),
+         (16, 20, 4, 128, 160, ((0, 28), (100, 51)), True)]
 
 
 @pytest.mark.parametrize("bits,heads,kvh,hd,seq,batches,rails", LINES)

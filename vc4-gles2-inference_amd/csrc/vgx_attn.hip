@@ -2074,7 +2074,8 @@ int launch_tile(vgx_attn* at, int layer, int pos, int ntok, const int16_t* qkv, 
     // against this kernel: heads of 64, q8 cache, 2 vectors 13.1 / 17.1, 4 16.8 / 17.4,
     // 6 22.2 / 17.7; q16 4 20.2 / 18.1, 6 26.7 / 18.4; heads of 96, q8 4 21.2 / 21.5, 6
     // 33.8 / 24.3; q16 4 25.3 / 22.8, 6 38.6 / 25.8; q16 at 250, 4 vectors: heads of 112
-    // 16.9 / 19.8, of 128 18.8 / 20.5.
+    // 16.9 / 19.8, of 128 18.8 / 20.5.  With 5 (20 heads over 4): q8 heads of 64 21.2 /
+    // 17.2, of 96 27.4 / 21.4, of 128 28.7 / 25.5; q16 of 128 32.4 / 28.3.
     if (g.hs * g.tq < (A.kv_bits == 16 && A.hd <= 96 ? 4 : 5)) return VGX_ESTATE;
     g.nby = (ntok + g.tq - 1) / g.tq;
     if (g.nby > 65535) return VGX_ESTATE;
