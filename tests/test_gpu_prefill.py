@@ -254,6 +254,43 @@ def test_gemm_routes(gpu, kind, rows, cols, ntok):
     W3.free()
 
 
+@pytest.mark.parametrize("kind", ["q8", "q4", "t3"])
+def test_split_k_under_capture(kind):
+    """A captured launch whose context has no split-K workspace yet runs whole, one
+    captured after an eager split splits; both graphs replay like the eager calls."""
+    from vgx import gpu as vg
+    g = vg.GPU(0)
+    rng = np.random.default_rng(19)
+    rows, cols, ntok = 96, 8192, 8
+    m = MK[kind](rng, rows, cols)
+    W = g.upload(m)
+    x, res = torch.zeros((ntok, cols), dtype=torch.int16, device="cuda"), dev(x_rows(rng, ntok, rows))
+    outs, graphs = [], []
+    for _ in range(2):
+        y = torch.zeros((ntok, rows), dtype=torch.int16, device="cuda")
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            g.use_torch_stream()
+            g.gemm(W, x, res=res, out=y)
+        g.use_torch_stream()
+        outs.append(y)
+        graphs.append(graph)
+        g.gemm(W, x, res=res)  # (allocates the workspace)
+    for _ in range(3):
+        xs = x_rows(rng, ntok, cols)
+        x.copy_(dev(xs))
+        want = np.stack([o.store(oracle_rowval(m, xs[t]), host(res)[t]) for t in range(ntok)])
+        assert np.array_equal(host(g.gemm(W, x, res=res)), want)
+        for y, graph in zip(outs, graphs):
+            y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(host(y), want)
+    W.free()
+    g.close()
+
+
 def test_gemm_past_one_grid_dimension(gpu):
     """More outputs than workgroups of 512 threads fit along x of a grid (2^32
     threads): 2,080 tokens of 2^22 rows, 17 GB, written over the residual."""
